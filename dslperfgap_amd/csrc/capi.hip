@@ -443,6 +443,72 @@ Geometry reduce_geometry(int64_t n, int vec, int64_t units) {
   return g;
 }
 
+// Launch shape of a middle-axis reduction over [outer, n, inner] (column tiles;
+// `esize` bytes per element).  More lines per unit (2^ty_log2) make more
+// workgroups of fewer rows per lane; fewer lines let a workgroup cover a wider
+// piece of each row.  MI355X, device time per call:
+//   lines until the launch has kColGrid workgroups, kColGridLarge from
+//   kColLargeBytes up: max bf16 64 x 2048 x 2048 at 8 / 16 / 32 lines 82 / 89 /
+//   99 us, mean fp32 512 x 256 x 512 at 4 / 32 lines 41.2 / 47.2 us, but max
+//   bf16 16 x 64 x 16384 at 4 / 8 lines 12.3 / 8.9 us and max fp16
+//   64 x 512 x 768 at 8 / 16 / 32 lines 15.4 / 13.0 / 12.5 us;
+//   the axis is split over workgroups, and the segments combined by a second
+//   launch, where even the most lines leave fewer than kColSplitGrid
+//   workgroups (kColGridLarge of a large launch, kColSplitGridNarrow of rows
+//   under 128 bytes) and kColSplitRows or more rows per lane: mean fp32
+//   1 x 8192 x 256 26 -> 6.9 us, 1 x 4096 x 4096 19.9 -> 15.8, max fp32
+//   1 x 16384 x 4096 53.9 -> 44.1, mean bf16 8 x 4096 x 2048 30.0 -> 24.2; but
+//   max bf16 16 x 2048 x 1024 at 256 workgroups 17.7, split 20.5, and of 16
+//   rows per lane max fp16 16 x 512 x 512 7.2, split 8.2.
+constexpr int64_t kColLargeBytes = int64_t(96) << 20;
+constexpr int64_t kColGrid = 1024;
+constexpr int64_t kColGridLarge = 512;
+constexpr int64_t kColSplitGrid = 256;
+constexpr int64_t kColSplitGridNarrow = 128;
+constexpr int64_t kColSplitTarget = 256;
+constexpr int64_t kColSplitRows = 64;
+constexpr int kColSplitLines = 16;
+
+ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int esize,
+                         bool can_split) {
+  ColGeometry c;
+  c.v = inner >= vn ? vn : 1;
+  const int64_t cv = (inner + c.v - 1) / c.v;
+  const int64_t bytes = mul_sat(mul_sat(outer, n), mul_sat(inner, esize));
+  const bool large = bytes >= kColLargeBytes;
+  // lanes per line: 8 (a 128-byte line of memory), or a narrow slab's whole row
+  c.cx = static_cast<int>(cv <= 12 ? cv : 8);
+  c.tiles = (cv + c.cx - 1) / c.cx;
+  auto grid_at = [&](int lines) {
+    const int64_t per_block = kColBlock / (c.cx * lines);
+    return (mul_sat(outer, c.tiles) + per_block - 1) / per_block;
+  };
+  int most = 1;  // lines: at least 4 rows each
+  while (most * 2 * c.cx <= kColBlock && int64_t(most) * 8 <= n) most *= 2;
+  int lines = std::min(most, 4);
+  while (lines < most && grid_at(lines) < (large ? kColGridLarge : kColGrid)) lines *= 2;
+  c.segs = 1;
+  if (can_split && n / lines >= kColSplitRows &&
+      grid_at(lines) < (cv < 8 ? kColSplitGridNarrow : large ? kColGridLarge : kColSplitGrid)) {
+    lines = c.cx >= 8 ? std::min(most, kColSplitLines) : most;
+    while (c.segs < kColMaxSegs && grid_at(lines) * c.segs < kColSplitTarget &&
+           n / (int64_t(c.segs) * 2 * lines) >= 8)
+      c.segs *= 2;
+  }
+  if (grid_at(lines) > kMaxWorkItems / kColBlock) {  // billions of columns: one lane each
+    lines = 1;
+    if (grid_at(lines) > kMaxWorkItems / kColBlock) {
+      c.tiles = cv;
+      c.cx = 1;
+    }
+  }
+  c.ty_log2 = __builtin_ctz(lines);
+  c.grid = grid_at(lines);
+  c.seg_n = static_cast<int>((n + c.segs - 1) / c.segs);
+  c.segs = c.seg_n > 0 ? static_cast<int>((n + c.seg_n - 1) / c.seg_n) : 1;
+  return c;
+}
+
 }  // namespace
 
 // function_for's cache: per device, an open-addressing table from kernel
@@ -1157,10 +1223,15 @@ int64_t split_entry_bytes(int op, int in_dtype) {
 
 int64_t vbh_reduce_workspace_bytes(int64_t outer, int64_t n, int64_t inner, int in_dtype,
                                    int op) {
-  if (op < 0 || op > 2 || !is_float(in_dtype) || inner != 1 || outer <= 0 || n <= 0 ||
+  if (op < 0 || op > 2 || !is_float(in_dtype) || inner <= 0 || outer <= 0 || n <= 0 ||
       n > kMaxCols)
     return 0;
   const int vn = 16 / elt_size(in_dtype);
+  if (inner > 1) {
+    if (mul_sat(outer, inner) > kMaxWorkItems / 256 * 256) return 0;
+    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), true);
+    return c.segs > 1 ? outer * inner * c.segs * (op == 0 ? 4 : 8) : 0;
+  }
   if (n % vn != 0 || g_tpr[VBH_OP_REDUCE].load() || g_block[VBH_OP_REDUCE].load()) return 0;
   const int segs = split_segments(outer, n / vn);
   return segs > 1 ? outer * segs * split_entry_bytes(op, in_dtype) : 0;
@@ -1185,8 +1256,8 @@ int vbh_reduce_fwd_ws(const void* x, void* values, void* indices, int64_t outer,
   const hipStream_t s = static_cast<hipStream_t>(stream);
   int64_t* idx = static_cast<int64_t*>(indices);
   Geometry g;
+  const int vn = 16 / elt_size(in_dtype);
   if (inner == 1) {
-    const int vn = 16 / elt_size(in_dtype);
     const bool vec_ok = n % vn == 0 && aligned16(x);
     const int64_t need = vbh_reduce_workspace_bytes(outer, n, inner, in_dtype, op);
     if (need > 0 && vec_ok && workspace != nullptr && workspace_bytes >= need &&
@@ -1202,14 +1273,14 @@ int vbh_reduce_fwd_ws(const void* x, void* values, void* indices, int64_t outer,
         float* means = static_cast<float*>(workspace);
         const Geometry g2 = reduce_geometry(segs, segs % 4 == 0 ? 4 : 1, outer);
         if (int rc = check_grid(outer, g2)) return rc;
-        e = launch_reduce(x, means, nullptr, units, seg_n, 1, in_dtype, kF32, 0, g1, s);
+        e = launch_reduce(x, means, nullptr, units, seg_n, in_dtype, kF32, 0, g1, s);
         if (e == hipSuccess)
-          e = launch_reduce(means, values, nullptr, outer, segs, 1, kF32, out_dtype, 0, g2, s);
+          e = launch_reduce(means, values, nullptr, outer, segs, kF32, out_dtype, 0, g2, s);
       } else {
         // segment (value, index) results, then the first maximal one per row
         int64_t* pidx = static_cast<int64_t*>(workspace);
         void* pvals = pidx + units;
-        e = launch_reduce(x, pvals, pidx, units, seg_n, 1, in_dtype, in_dtype, 1, g1, s);
+        e = launch_reduce(x, pvals, pidx, units, seg_n, in_dtype, in_dtype, 1, g1, s);
         if (e == hipSuccess)
           e = launch_reduce_combine(pvals, pidx, values, idx, outer, segs, seg_n, in_dtype, op,
                                     s);
@@ -1220,10 +1291,18 @@ int vbh_reduce_fwd_ws(const void* x, void* values, void* indices, int64_t outer,
     g = reduce_geometry(n, vec_ok || mis_ok ? vn : 1, outer);
     if (mis_ok && !use_mis(g, vn)) g = reduce_geometry(n, 1, outer);
     if (int rc = check_grid(outer, g)) return rc;
-  } else if (mul_sat(outer, inner) > kMaxWorkItems / 256 * 256) {
-    return fail(VBH_E_RANGE, "reduce: outer * inner too large");
+  } else {
+    if (mul_sat(outer, inner) > kMaxWorkItems / 256 * 256)
+      return fail(VBH_E_RANGE, "reduce: outer * inner too large");
+    const int64_t need = vbh_reduce_workspace_bytes(outer, n, inner, in_dtype, op);
+    const bool split = need > 0 && workspace != nullptr && workspace_bytes >= need &&
+                       aligned16(workspace);
+    return hip_status(launch_reduce_cols(x, values, idx, split ? workspace : nullptr, outer,
+                                         static_cast<int>(n), inner, in_dtype, out_dtype, op,
+                                         col_geometry(outer, n, inner, vn, elt_size(in_dtype), split), s),
+                      "reduce launch");
   }
-  return hip_status(launch_reduce(x, values, idx, outer, static_cast<int>(n), inner, in_dtype,
+  return hip_status(launch_reduce(x, values, idx, outer, static_cast<int>(n), in_dtype,
                                   out_dtype, op, g, s),
                     "reduce launch");
 }

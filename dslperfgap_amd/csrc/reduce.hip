@@ -4,8 +4,9 @@
 //   inner == 1 (last axis): `tpr` lanes own one row and stream it with 16-byte
 //   loads (nothing per element is written, so the row is never held in
 //   registers and any n works), then all-reduce across the group.
-//   inner > 1: one lane per (outer, inner) column loops over n; consecutive
-//   lanes read consecutive inner indices, so every access is coalesced.
+//   inner > 1: column tiles (col_lane): each lane owns the columns of one
+//   16-byte vector and takes every 2^ty_log2-th row, the lines of lanes are
+//   combined through LDS; few columns split the axis over workgroups.
 // Each input element is read once; one value (and/or index) per output is
 // written.
 //
@@ -15,6 +16,8 @@
 // int64 indices (ViperBench/argmax/pytorch_impl.py:4-8).  NaN counts as the
 // largest value and ties resolve to the smallest index, so the first maximal
 // (or first NaN) position is returned.
+#include <limits.h>
+
 #include "vbh_device.h"
 #include "vbh_launch.h"
 
@@ -339,42 +342,197 @@ __global__ __launch_bounds__(256) void reduce_combine_vi(const T* __restrict__ p
   if (VBH_IN_SPAN(si, idx + row, sizeof(int64_t))) idx[row] = best.i;
 }
 
-template <typename Ti, typename To, int OP>
-__global__ __launch_bounds__(256) void reduce_cols(const Ti* __restrict__ x,
-                                                   void* __restrict__ vals,
-                                                   int64_t* __restrict__ idx, int64_t outer,
-                                                   int n, int64_t inner) {
-  const int64_t col = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (col >= outer * inner) return;
-  const int64_t o = col / inner;
-  const int64_t c = col - o * inner;
-  const Ti* xc = x + o * n * inner + c;
+// Middle axis: column tiles (col_lane in vbh_device.h) of kColBlock lanes.
+// PART (first stage of a split axis, grid.y segments of seg_n rows): each
+// column's fp32 sum or value goes to pv[seg * columns + column] and its row to
+// pi; else the result to vals / idx.
+//
+// Bound by memory: every element is read once, eight rows (128 bytes of loads)
+// per lane in flight.  The kernel it replaced ran one lane per column with one
+// element in flight and left most CUs idle.  MI355X, time per call before ->
+// after (the bytes at the copy's rate): max fp16 64 x 512 x 768 149 -> 12.1 us
+// (7.0), mean fp32 512 x 32 x 4096 77 -> 44 (38), max fp16 20 x 200 x 20000 111
+// -> 36 (23), mean fp32 8192 x 64 x 49 34 -> 16.8 (14), max bf16 4096 x 2 x 4096
+// 78 -> 38 (32).  Max and argmax stay up to 2 us behind the mean: five VALU
+// instructions per element (convert, two compares, two selects).  Results go
+// through LDS to the lanes that write them, so that stores of consecutive
+// columns coalesce (straight from the lanes, the int64 indices of one lane are
+// 64 bytes apart: max fp32 3375 x 3 x 512 12.9 against 8.7 us).
+template <typename Ti, typename To, int V, int OP, bool PART>
+__global__ __launch_bounds__(kColBlock) void reduce_cols(
+    const Ti* __restrict__ x, void* __restrict__ vals, int64_t* __restrict__ idx,
+    float* __restrict__ pv, int* __restrict__ pi, int64_t outer, int n, int64_t inner, int cx,
+    int ty_log2, uint32_t tiles, int seg_n) {
+  typedef typename Raw<Ti, V>::type RT;
+  constexpr int U = 8;  // rows in flight per lane
+  constexpr int B = kColBlock;
+  // a workgroup's columns side by side, line after line
+  __shared__ __align__(16) float lds_v[V * B];
+  __shared__ __align__(16) int lds_i[OP == 0 ? 4 : V * B];
+  // per vector of the workgroup: its first output times 8, plus how many of its
+  // columns the vector before it writes
+  __shared__ int64_t lds_out[B];
+  const ColLane L = col_lane<V>(outer, inner, cx, ty_log2, tiles);
+  const int64_t cols = outer * inner;
   const Span sx = VBH_SPAN(x, outer * n * inner);
-  const Span sv = VBH_SPAN(static_cast<To*>(vals), outer * inner), si = VBH_SPAN(idx, outer * inner);
-  auto xat = [&](int r) {
-    float v;
-    load_f32<Ti, 1>(xc + r * inner, &v, sx);
-    return v;
-  };
-  if constexpr (OP == 0) {
-    float s = 0.f;
-    for (int r = 0; r < n; ++r) s += xat(r);
-    write_result<To, 1, OP>(vals, idx, col, s, 0, n, sv, si);
-  } else {
-    ValIdx best{kNegInf, n};
-    for (int r = 0; r < n; ++r) {
-      const float v = xat(r);
-      if (better(v, r, best.v, best.i)) best = ValIdx{v, r};
-    }
-    write_result<To, 1, OP>(vals, idx, col, best.v, best.i, n, sv, si);
+  const int seg = static_cast<int>(blockIdx.y);
+  const int r0 = PART ? seg * seg_n : 0;
+  const int len = PART ? min(n - r0, seg_n) : n;  // rows of this segment
+  const int rows = L.live && L.ty < len ? ((len - L.ty - 1) >> ty_log2) + 1 : 0;  // the lane's
+  const int64_t step = inner << ty_log2;
+  const Ti* p = x + (L.o * n + r0 + L.ty) * inner + L.col;
+
+  float a[V];  // the lane's sums, or its best values
+  int at[OP == 0 ? 1 : V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) a[k] = OP == 0 ? 0.f : kNegInf;
+  if constexpr (OP != 0) {
+    // a lane whose values are all -inf has its first row, one without rows none
+#pragma unroll
+    for (int k = 0; k < V; ++k) at[k] = rows > 0 ? r0 + L.ty : INT_MAX;
   }
+  auto take = [&](const RT& v, int r) {
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const float f = raw_at<Ti, V>(v, k);
+      if constexpr (OP == 0) {
+        a[k] += f;
+      } else {
+        // larger, or the column's first NaN
+        const bool win = !(f <= a[k]) && a[k] == a[k];
+        a[k] = win ? f : a[k];
+        at[k] = win ? r : at[k];
+      }
+    }
+  };
+  int i = 0;
+  for (; rows - i >= U; i += U, p += U * step) {
+    RT v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = load_any<Ti, V>(p + u * step, sx);
+#pragma unroll
+    for (int u = 0; u < U; ++u) take(v[u], r0 + L.ty + ((i + u) << ty_log2));
+  }
+  if (i < rows) {
+    RT v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u < rows) v[u] = load_any<Ti, V>(p + u * step, sx);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u < rows) take(v[u], r0 + L.ty + ((i + u) << ty_log2));
+  }
+  // Through LDS, so that consecutive lanes write consecutive columns: each of
+  // the workgroup's W columns is combined by `parts` lanes over its lines,
+  // then by one over their results.
+  const int W = L.per_block * cx * V;
+  const int TY = 1 << ty_log2;
+  const int t = static_cast<int>(threadIdx.x);
+  if (L.sub < L.per_block) {
+    const int vec = L.sub * cx + L.c;
+    const int j = L.ty * W + vec * V;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      lds_v[j + k] = a[k];
+      if constexpr (OP != 0) lds_i[j + k] = at[k];
+    }
+    if (L.ty == 0) lds_out[vec] = L.live ? (L.o * inner + L.col) * 8 + L.shared : -1;
+  }
+  __syncthreads();
+  auto gather = [&](int j, int stride, int count) {  // over lds[j], lds[j + stride], ...
+    ValIdx r{lds_v[j], OP == 0 ? 0 : lds_i[OP == 0 ? 0 : j]};
+    for (int s = 1; s < count; ++s) {
+      j += stride;
+      if constexpr (OP == 0) r.v += lds_v[j];
+      else r = pick(r, ValIdx{lds_v[j], lds_i[j]});
+    }
+    return r;
+  };
+  int lines = TY;
+  if (TY > 2 && W * 2 <= B) {
+    int parts = TY >> 1;  // at least two lines each
+    while (parts * W > B) parts >>= 1;
+    const int part = t / W, j = t - part * W;
+    ValIdx r{0.f, 0};
+    const int per = TY / parts;  // powers of two
+    if (part < parts) r = gather(part * per * W + j, W, per);
+    __syncthreads();
+    if (part < parts) {
+      lds_v[part * W + j] = r.v;
+      if constexpr (OP != 0) lds_i[part * W + j] = r.i;
+    }
+    __syncthreads();
+    lines = parts;
+  }
+  const Span sv = VBH_SPAN(static_cast<To*>(vals), PART ? 0 : cols),
+             si = VBH_SPAN(idx, PART ? 0 : cols);
+  const Span spv = VBH_SPAN(pv, PART ? cols * gridDim.y : 0),
+             spi = VBH_SPAN(pi, PART ? cols * gridDim.y : 0);
+  for (int j = t; j < W; j += B) {
+    const int64_t base = lds_out[j / V];
+    const int k = j & (V - 1);
+    if (base < 0 || k < static_cast<int>(base & 7)) continue;
+    const int64_t out = (base >> 3) + k;
+    const ValIdx r = gather(j, W, lines);
+    if constexpr (PART) {
+      const int64_t q = static_cast<int64_t>(seg) * cols + out;
+      store_from_f32<float, 1>(pv + q, &r.v, spv);
+      if constexpr (OP != 0)
+        if (VBH_IN_SPAN(spi, pi + q, sizeof(int))) pi[q] = r.i;
+    } else {
+      write_result<To, 1, OP>(vals, idx, out, r.v, r.i, n, sv, si);
+    }
+  }
+}
+
+// Second stage of a split middle axis: kCombineParts lanes per column, each
+// over every kCombineParts-th of its `segs` (<= 64) partial results, then one.
+constexpr int kCombineParts = 8;
+constexpr int kCombineCols = kColBlock / kCombineParts;
+
+template <typename To, int OP>
+__global__ __launch_bounds__(kColBlock) void reduce_cols_combine(
+    const float* __restrict__ pv, const int* __restrict__ pi, void* __restrict__ vals,
+    int64_t* __restrict__ idx, int64_t cols, int n, int segs) {
+  constexpr int M = kColMaxSegs / kCombineParts;
+  __shared__ float lds_v[kColBlock];
+  __shared__ int lds_i[kColBlock];
+  const int t = static_cast<int>(threadIdx.x);
+  const int j = t % kCombineCols, part = t / kCombineCols;
+  const int64_t col = static_cast<int64_t>(blockIdx.x) * kCombineCols + j;
+  const Span sp = VBH_SPAN(pv, cols * segs), spi = VBH_SPAN(pi, cols * segs);
+  const Span sv = VBH_SPAN(static_cast<To*>(vals), cols), si = VBH_SPAN(idx, cols);
+  ValIdx w[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const int s = part + m * kCombineParts;
+    w[m] = ValIdx{OP == 0 ? 0.f : kNegInf, INT_MAX};
+    if (s < segs && col < cols) {
+      const int64_t q = s * cols + col;
+      load_f32<float, 1>(pv + q, &w[m].v, sp);
+      if constexpr (OP != 0) w[m].i = VBH_IN_SPAN(spi, pi + q, sizeof(int)) ? pi[q] : 0;
+    }
+  }
+  auto fold = [](ValIdx a, ValIdx b) {
+    if constexpr (OP == 0) return ValIdx{a.v + b.v, 0};
+    else return pick(a, b);
+  };
+#pragma unroll
+  for (int m = 1; m < M; ++m) w[0] = fold(w[0], w[m]);
+  lds_v[t] = w[0].v;
+  lds_i[t] = w[0].i;
+  __syncthreads();
+  if (part != 0 || col >= cols) return;
+#pragma unroll
+  for (int q = 1; q < kCombineParts; ++q)
+    w[0] = fold(w[0], ValIdx{lds_v[q * kCombineCols + j], lds_i[q * kCombineCols + j]});
+  write_result<To, 1, OP>(vals, idx, col, w[0].v, w[0].i, n, sv, si);
 }
 
 }  // namespace
 
-hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer, int n,
-                         int64_t inner, int idt, int odt, int op, const Geometry& g,
-                         hipStream_t s) {
+hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer, int n, int idt,
+                         int odt, int op, const Geometry& g, hipStream_t s) {
   hipError_t err = hipErrorInvalidValue;
   auto body = [&](auto ti, auto to) {
     using Ti = typename decltype(ti)::type;
@@ -382,19 +540,13 @@ hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer,
     constexpr int VN = Vec<Ti>::n;
     auto go = [&](auto opc) {
       constexpr int OP = decltype(opc)::value;
-      if (inner == 1) {
-        auto launch = [&](auto kern) {
-          launch_kernel(kern, dim3(grid_for(outer, g)), dim3(g.block), 0, s,
-                             static_cast<const Ti*>(x), vals, idx, outer, n, g.tpr);
-        };
-        if (g.v == 1) launch(reduce_rows<Ti, To, 1, OP, false>);
-        else if (g.mis) launch(reduce_rows<Ti, To, VN, OP, true>);
-        else launch(reduce_rows<Ti, To, VN, OP, false>);
-      } else {
-        const int64_t cols = outer * inner;
-        launch_kernel((reduce_cols<Ti, To, OP>), dim3((cols + 255) / 256), dim3(256), 0, s,
-                           static_cast<const Ti*>(x), vals, idx, outer, n, inner);
-      }
+      auto launch = [&](auto kern) {
+        launch_kernel(kern, dim3(grid_for(outer, g)), dim3(g.block), 0, s,
+                           static_cast<const Ti*>(x), vals, idx, outer, n, g.tpr);
+      };
+      if (g.v == 1) launch(reduce_rows<Ti, To, 1, OP, false>);
+      else if (g.mis) launch(reduce_rows<Ti, To, VN, OP, true>);
+      else launch(reduce_rows<Ti, To, VN, OP, false>);
       err = hipGetLastError();
     };
     if (op == 0) go(std::integral_constant<int, 0>{});
@@ -405,9 +557,53 @@ hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer,
     dispatch_float_type(idt, [&](auto t) { body(t, t); });
   } else if (op == 0 && odt == kF32 && (idt == kF16 || idt == kBF16)) {
     dispatch_float_type(idt, [&](auto t) { body(t, TypeTag<float>{}); });
-  } else if (op == 0 && idt == kF32 && (odt == kF16 || odt == kBF16) && inner == 1) {
+  } else if (op == 0 && idt == kF32 && (odt == kF16 || odt == kBF16)) {
     // second stage of a split mean: fp32 segment means in, the output type out
     dispatch_float_type(odt, [&](auto t) { body(TypeTag<float>{}, t); });
+  }
+  return err;
+}
+
+hipError_t launch_reduce_cols(const void* x, void* vals, int64_t* idx, void* parts,
+                              int64_t outer, int n, int64_t inner, int idt, int odt, int op,
+                              const ColGeometry& c, hipStream_t s) {
+  hipError_t err = hipErrorInvalidValue;
+  const int64_t cols = outer * inner;
+  float* pv = static_cast<float*>(parts);
+  int* pi = pv == nullptr ? nullptr : reinterpret_cast<int*>(pv + cols * c.segs);
+  auto body = [&](auto ti, auto to) {
+    using Ti = typename decltype(ti)::type;
+    using To = typename decltype(to)::type;
+    auto go = [&](auto opc, auto vc) {
+      constexpr int OP = decltype(opc)::value;
+      constexpr int V = decltype(vc)::value;
+      auto launch = [&](auto kern) {
+        launch_kernel(kern, dim3(static_cast<uint32_t>(c.grid), static_cast<uint32_t>(c.segs)),
+                      dim3(kColBlock), 0, s, static_cast<const Ti*>(x), vals, idx, pv, pi, outer,
+                      n, inner, c.cx, c.ty_log2, static_cast<uint32_t>(c.tiles), c.seg_n);
+      };
+      if (c.segs > 1) {
+        launch(reduce_cols<Ti, To, V, OP, true>);
+        launch_kernel((reduce_cols_combine<To, OP>),
+                      dim3(static_cast<uint32_t>((cols + kCombineCols - 1) / kCombineCols)),
+                      dim3(kColBlock), 0, s, pv, pi, vals, idx, cols, n, c.segs);
+      } else {
+        launch(reduce_cols<Ti, To, V, OP, false>);
+      }
+      err = hipGetLastError();
+    };
+    auto by_op = [&](auto vc) {
+      if (op == 0) go(std::integral_constant<int, 0>{}, vc);
+      else if (op == 1) go(std::integral_constant<int, 1>{}, vc);
+      else go(std::integral_constant<int, 2>{}, vc);
+    };
+    if (c.v == 1) by_op(std::integral_constant<int, 1>{});
+    else by_op(std::integral_constant<int, Vec<Ti>::n>{});
+  };
+  if (idt == odt) {
+    dispatch_float_type(idt, [&](auto t) { body(t, t); });
+  } else if (op == 0 && odt == kF32 && (idt == kF16 || idt == kBF16)) {
+    dispatch_float_type(idt, [&](auto t) { body(t, TypeTag<float>{}); });
   }
   return err;
 }

@@ -186,6 +186,81 @@ __device__ __forceinline__ void store_raw(T* __restrict__ p, const float* o, con
   else *q = r;
 }
 
+// The same 16-byte accesses at any element-aligned address (global accesses of
+// several dwords take any byte address on gfx9 under the unaligned access mode
+// the HSA ABI turns on), for tiles of rows that do not start at a vector
+// boundary.  V elements need not fill 16 bytes.
+template <typename T, int V> struct RawAny {
+  typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+};
+template <typename T> struct RawAny<T, 1> { typedef T type; };
+
+template <typename T, int V>
+__device__ __forceinline__ typename Raw<T, V>::type load_any(const T* __restrict__ p,
+                                                             const Span& s) {
+  typedef typename RawAny<T, V>::type A;
+  if (!VBH_IN_SPAN(s, p, V * sizeof(T))) return typename Raw<T, V>::type{};
+  return __builtin_nontemporal_load(reinterpret_cast<const A*>(p));
+}
+
+template <typename T, int V>
+__device__ __forceinline__ void store_any(T* __restrict__ p, const float* o, const Span& s) {
+  typedef typename RawAny<T, V>::type A;
+  if (!VBH_IN_SPAN(s, p, V * sizeof(T))) return;
+  A r;
+  if constexpr (V == 1) {
+    r = static_cast<T>(o[0]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < V; ++k) r[k] = static_cast<T>(o[k]);
+  }
+  __builtin_nontemporal_store(r, reinterpret_cast<A*>(p));
+}
+
+// ---------------------------------------------------------------------------
+// column tiles: reductions over the middle axis of a contiguous
+// [outer, n, inner] tensor
+//
+// A unit is one column tile of one outer slab: cx lanes side by side, each
+// with V consecutive inner indices, so that a row of the tile is one
+// contiguous piece of memory.  Every unit is worked on by 2^ty_log2 such lines
+// of lanes: line ty takes rows ty, ty + 2^ty_log2, ..., and the lines' results
+// are combined through LDS.  A workgroup holds blockDim.x / (cx << ty_log2)
+// units, lanes past them idle.  The last tile's last vector is moved back to
+// end at the slab's edge where inner is no multiple of V; the columns it then
+// shares with the vector before it (`shared`) are written by that one.
+// ---------------------------------------------------------------------------
+struct ColLane {
+  int c, ty;     // place in the line, line
+  int sub;       // unit of the workgroup
+  int per_block; // units a workgroup holds
+  int64_t o;     // outer index
+  int64_t col;   // first inner index of the lane's vector
+  int shared;    // leading columns of it that the vector before it writes
+  bool live;     // the lane has a vector
+};
+
+template <int V>
+__device__ __forceinline__ ColLane col_lane(int64_t outer, int64_t inner, int cx, int ty_log2,
+                                            uint32_t tiles) {
+  ColLane L;
+  const int t = static_cast<int>(threadIdx.x);
+  const int q = t / cx;
+  L.c = t - q * cx;
+  L.ty = q & ((1 << ty_log2) - 1);
+  L.sub = q >> ty_log2;
+  L.per_block = static_cast<int>(blockDim.x) / (cx << ty_log2);
+  const uint32_t u = static_cast<uint32_t>(blockIdx.x) * static_cast<uint32_t>(L.per_block) +
+                     static_cast<uint32_t>(L.sub);
+  const uint32_t o = tiles == 1 ? u : u / tiles;
+  L.o = o;
+  const int64_t first = (static_cast<int64_t>(u - o * tiles) * cx + L.c) * V;
+  L.live = L.sub < L.per_block && L.o < outer && first < inner;
+  L.col = first + V <= inner ? first : inner - V;
+  L.shared = static_cast<int>(first - L.col);
+  return L;
+}
+
 // ---------------------------------------------------------------------------
 // output store policies of the row kernels
 // ---------------------------------------------------------------------------

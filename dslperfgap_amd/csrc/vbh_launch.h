@@ -276,9 +276,29 @@ struct CeBwdArgs {
 constexpr int kCeBwdLanes = 256;
 hipError_t launch_cross_entropy_bwd(const CeBwdArgs& a, hipStream_t s);
 
-hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer, int n,
-                         int64_t inner, int idt, int odt, int op, const Geometry& g,
-                         hipStream_t s);
+hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer, int n, int idt,
+                         int odt, int op, const Geometry& g, hipStream_t s);
+
+// Launch shape of a kernel over column tiles (col_lane in vbh_device.h): `v`
+// elements per lane, `cx` lanes per line of a tile, 2^ty_log2 lines per unit,
+// `tiles` units per outer slab, `grid` workgroups, the axis cut into `segs`
+// segments of seg_n rows (the last one shorter).
+constexpr int kColBlock = 256;
+constexpr int kColMaxSegs = 64;
+struct ColGeometry {
+  int v = 1;
+  int cx = 1;
+  int ty_log2 = 0;
+  int64_t tiles = 1;
+  int64_t grid = 1;
+  int segs = 1;
+  int seg_n = 0;
+};
+// Reduction over the middle axis.  With c.segs > 1, `parts` holds
+// outer * inner * segs fp32 results, and as many int32 rows for max / argmax.
+hipError_t launch_reduce_cols(const void* x, void* vals, int64_t* idx, void* parts,
+                              int64_t outer, int n, int64_t inner, int idt, int odt, int op,
+                              const ColGeometry& c, hipStream_t s);
 // Second stage of a split max (op 1) / argmax (op 2): per row, the winner of
 // `segs` segment results (values of type `dt`, int64 segment-local indices).
 hipError_t launch_reduce_combine(const void* pvals, const int64_t* pidx, void* vals, int64_t* idx,

@@ -232,7 +232,9 @@ int vbh_reduce_fwd(const void* x, void* values, void* indices, int64_t outer, in
 /* vbh_reduce_fwd with a caller-provided device workspace (16-byte aligned):
  * last-axis reductions (inner == 1) of few long rows are split into segments
  * reduced in parallel, then combined per row (the mean of the equal segments'
- * fp32 means; the first maximal segment result, NaN largest).  Workspace
+ * fp32 means; the first maximal segment result, NaN largest); middle-axis ones
+ * of few columns and many rows into segments of rows, whose fp32 sums (or
+ * values and rows) are combined per column.  Workspace
  * size, fallback and reuse as for vbh_logsumexp_fwd_ws, with
  * vbh_reduce_workspace_bytes.  No reference counterpart: torch.mean / max /
  * argmax (the goldens above) choose their own split internally. */

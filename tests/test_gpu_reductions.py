@@ -292,3 +292,49 @@ def test_misaligned_rows_reductions(dtype):
         _same(argmax(xd, 1), ref.argmax(x, 1), "argmax " + what)
         xm = torch.randn(rows, n, generator=_g(710 + n)).to(dtype) + 2.0
         _close(mean_reduction(xm.to(DEV), 1), ref.mean_reduction(xm, 1), "mean " + what)
+
+
+# ---------------------------------------------------------------------------
+# middle and first axes: column tiles, split axes
+# ---------------------------------------------------------------------------
+def _special(x):
+    """Ties, a NaN after a larger value, two NaNs, infinities and an all -inf column."""
+    c, n = x.shape[2], x.shape[1]
+    x[0, n // 2, 0] = x[0, n - 1, 0] = 30.0
+    if c > 1 and n > 2:
+        x[0, 0, 1] = 40.0
+        x[0, n - 1, 1] = x[0, n - 2, 1] = float("nan")
+    x[-1, :, c - 1] = float("-inf")
+    if c > 3:
+        x[-1, n // 3, c - 2] = float("inf")
+        x[-1, :, c - 3] = torch.finfo(x.dtype).min
+    return x
+
+
+COL_SHAPES = [(3, n, i) for n in (1, 2, 7, 8, 33) for i in (2, 3, 7, 8, 9, 13, 64, 101)] + [
+    (1, 257, 65), (70, 5, 12), (2, 300, 97), (5, 1000, 31), (1, 3000, 2), (600, 40, 68)]
+# the axis split over workgroups (the last segment shorter in some)
+COL_SPLIT_SHAPES = [(1, 4100, 264), (1, 9001, 33), (2, 20000, 12), (1, 50000, 3)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", COL_SHAPES + COL_SPLIT_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_middle_axis_column_tiles(shape, dtype):
+    """Max and argmax exactly.  The mean within n additions of fp32 (at most n *
+    2^-24 of the mean magnitude, far below TOL for these n) and its rounding to
+    the output type."""
+    code = {torch.float32: _lib.F32, torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}[dtype]
+    split = _lib.reduce_workspace_bytes(*shape, code, _lib.REDUCE_MEAN) > 0
+    assert split == (shape in COL_SPLIT_SHAPES)
+    x = torch.randn(shape, generator=_g(310)).to(dtype)
+    _close(mean_reduction(x.to(DEV), 1), ref.mean_reduction(x, 1), "mean")
+    if dtype != torch.float32:
+        _close(mean_reduction(x.to(DEV), 1, False, torch.float32),
+               ref.mean_reduction(x, 1, False, torch.float32), "mean to fp32")
+    x = _special(x)
+    xd = x.to(DEV)
+    v, i = max_reduction(xd, 1)
+    rv, ri = ref.max_reduction(x, 1)
+    _same(v, rv, "values")
+    _same(i, ri, "indices")
+    _same(argmax(xd, 1), ref.argmax(x, 1), "argmax")
