@@ -509,6 +509,57 @@ ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int es
   return c;
 }
 
+// Launch shape of a middle-axis softmax over [outer, n, inner] (esize / osize
+// bytes per element of input and output).  8 lanes per line (a 128-byte line of
+// memory), 16 where a vector is 8 bytes of input or a lane holds the whole axis;
+// 4, or 2, where that leaves
+// fewer than kSmColUnits units, though two units then fetch each line.  MI355X,
+// log_softmax over the middle axis, us: bf16 -> fp32 16 x 64 x 16384 at 8 / 16
+// lanes 22.8 / 18.9; bf16 8 x 1000 x 1024 (128 units) at 8 / 4 19.4 / 15.5,
+// bf16 4 x 4096 x 1024 60 / 33.5, but fp32 8 x 2000 x 1024 (256 units)
+// 27.7 / 42.
+// Rows per lane: up to a wave per unit 4 or 8, then 16 in 256-lane workgroups
+// (fp16 64 x 512 x 768: 19.1, 8 rows in 1024 lanes 32.4; fp32 64 x 150 x 2048
+// 30.9 against 32.9), 4 while the launch has fewer than 512 workgroups, 8 and
+// 16 in 1024 lanes for longer axes (fp32 8 x 1000 x 1024: 15.5, 16 rows 17.2).
+// Axes that do not fit at 8 lanes stream (fp32 2 x 4096 x 8192: 170, 4 lanes of
+// 16 rows 223).
+constexpr int64_t kSmColUnits = 192;
+
+ColGeometry softmax_col_geometry(int64_t outer, int64_t n, int64_t inner, int esize, int osize) {
+  ColGeometry c;
+  const int vn = 16 / std::max(esize, osize);
+  c.v = inner >= vn ? vn : 1;
+  const int64_t cv = (inner + c.v - 1) / c.v;
+  auto lines_for = [&](int rows) {  // a unit has 16 lanes or more
+    return std::max(std::max(16 / c.cx, 1), pow2ceil((n + rows - 1) / rows));
+  };
+  auto fits = [&](int rows, int block) { return int64_t(lines_for(rows)) * c.cx <= block; };
+  auto units = [&] { return mul_sat(outer, (cv + c.cx - 1) / c.cx); };
+  c.cx = 16;
+  if (n > 4 && (c.v * esize == 16 || !fits(16, kColBlock) || units() < kSmColUnits))
+    c.cx = 8;
+  if (n > kWave && units() < kSmColUnits) c.cx = 4;
+  if (c.cx == 4 && !fits(16, kMaxBlock) && units() < kSmColUnits) c.cx = 2;
+  c.cx = static_cast<int>(std::min<int64_t>(pow2ceil(cv), c.cx));
+  c.tiles = (cv + c.cx - 1) / c.cx;
+  c.block = fits(16, kColBlock) ? kColBlock : kMaxBlock;
+  if (c.block == kColBlock) {
+    const int wave_lines = std::max(kWave / c.cx, 1);
+    c.rows = lines_for(4) <= wave_lines ? 4 : lines_for(8) <= wave_lines ? 8 : 16;
+    if (c.rows > 4 && fits(4, kColBlock) &&
+        mul_sat(units(), int64_t(lines_for(c.rows)) * c.cx) < 512 * kColBlock)
+      c.rows = 4;
+  } else {
+    c.rows = fits(8, kMaxBlock) ? 8 : fits(16, kMaxBlock) ? 16 : 0;
+  }
+  const int lines = c.rows > 0 ? lines_for(c.rows) : kMaxBlock / c.cx;
+  c.ty_log2 = __builtin_ctz(lines);
+  const int64_t per_block = c.block / (c.cx * lines);
+  c.grid = (units() + per_block - 1) / per_block;
+  return c;
+}
+
 }  // namespace
 
 // function_for's cache: per device, an open-addressing table from kernel
@@ -933,9 +984,25 @@ int vbh_softmax_dim_fwd(const void* x, void* y, int64_t outer, int64_t n, int64_
   if (!x || !y) return fail(VBH_E_INVALID, "softmax_dim: null pointer");
   if (mul_sat(outer, inner) > kMaxWorkItems / 256 * 256)
     return fail(VBH_E_RANGE, "softmax_dim: outer * inner too large");
-  return hip_status(launch_softmax_dim(x, y, outer, static_cast<int>(n), inner, in_dtype,
-                                       out_dtype, log_mode, static_cast<hipStream_t>(stream)),
-                    "softmax_dim launch");
+  const int esize = elt_size(in_dtype), osize = elt_size(out_dtype);
+  const ColGeometry c = softmax_col_geometry(outer, n, inner, esize, osize);
+  // billions of columns: as many launches as keep each under 2^32 work-items
+  const int64_t grid_max = kMaxWorkItems / c.block;
+  const int64_t pieces = (c.grid + grid_max - 1) / grid_max;
+  const int64_t piece = (outer + pieces - 1) / pieces;
+  for (int64_t o = 0; o < outer; o += piece) {
+    const int64_t at = o * n * inner;
+    const int64_t count = std::min(piece, outer - o);
+    if (int rc = hip_status(
+            launch_softmax_dim(static_cast<const char*>(x) + at * esize,
+                               static_cast<char*>(y) + at * osize, count, static_cast<int>(n),
+                               inner, in_dtype, out_dtype, log_mode,
+                               pieces == 1 ? c : softmax_col_geometry(count, n, inner, esize, osize),
+                               static_cast<hipStream_t>(stream)),
+            "softmax_dim launch"))
+      return rc;
+  }
+  return 0;
 }
 
 int64_t vbh_logsumexp_workspace_bytes(int64_t rows, int64_t cols, int in_dtype) {

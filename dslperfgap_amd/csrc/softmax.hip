@@ -6,9 +6,8 @@
 // exp(x - max), and writes the row once.
 // Streaming path (rows wider than the register budget): one workgroup per row,
 // online (max, rescaled sum) statistics pass, then an output pass.
-// Middle-axis path: contiguous [outer, n, inner] reduced over n; one thread per
-// (outer, inner) column, consecutive threads on consecutive inner indices so
-// every access is coalesced.
+// Middle-axis path: contiguous [outer, n, inner] reduced over n, in column
+// tiles: each lane owns the columns of one 16-byte vector and some of the rows.
 //
 // Semantics: ViperBench/softmax/pytorch_impl.py:4-6 (F.softmax, dim=-1),
 // ViperBench/log_softmax/pytorch_impl.py:4-8 (F.log_softmax(x, dim, dtype)),
@@ -477,38 +476,210 @@ __global__ __launch_bounds__(kMaxBlock) void logsumexp_stream(const Ti* __restri
 }
 
 // ---------------------------------------------------------------------------
-// middle axis: [outer, n, inner], reduce over n
+// middle axis: [outer, n, inner], reduce over n, in column tiles (col_lane in
+// vbh_device.h)
+//
+// The lanes of a unit lie line after line, so a column's values sit in every
+// cx-th lane: cx is a power of two up to kColMaxLanes and a unit has 16 lanes
+// or more, and the lines are all-reduced by row rotations and permlane swaps
+// in a wave, and through LDS over a unit's waves.
 // ---------------------------------------------------------------------------
-template <typename Ti, typename To, bool LOG>
-__global__ __launch_bounds__(256) void softmax_mid(const Ti* __restrict__ x,
-                                                   To* __restrict__ y, int64_t outer, int n,
-                                                   int64_t inner) {
-  const int64_t col = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (col >= outer * inner) return;
-  const int64_t o = col / inner;
-  const int64_t i = col - o * inner;
-  const Ti* xc = x + o * n * inner + i;
-  To* yc = y + o * n * inner + i;
-  const Span sx = VBH_SPAN(x, outer * n * inner), sy = VBH_SPAN(y, outer * n * inner);
-  auto xat = [&](int r) {
-    const Ti* p = xc + r * inner;
-    return VBH_IN_SPAN(sx, p, sizeof(Ti)) ? static_cast<float>(*p) : 0.f;
-  };
-  float m = kNegInf;
-  for (int r = 0; r < n; ++r) m = fmaxf(m, xat(r));
-  float s = 0.f;
-  for (int r = 0; r < n; ++r) s += fast_exp(xat(r) - m);
-  if constexpr (LOG) {
-    const float ls = fast_log(s);
-    for (int r = 0; r < n; ++r) {
-      const float out = (xat(r) - m) - ls;
-      store_from_f32<To, 1>(yc + r * inner, &out, sy);
-    }
+constexpr int kColMaxLanes = 16;
+
+// All-reduce over the lines of a 16-lane row (a unit of `lanes` >= 16 lanes, cx
+// per line): after the step by 2s lanes the values repeat every 2s lanes, so a
+// rotation by s brings the partner lane ^ s.
+template <class Op>
+__device__ __forceinline__ float lines_allreduce(float v, int cx, int lanes) {
+  if (cx <= 8) v = Op::apply(v, dpp<0x128>(v));  // row_ror:8
+  if (cx <= 4) v = Op::apply(v, dpp<0x124>(v));
+  if (cx <= 2) v = Op::apply(v, dpp<0x122>(v));
+  if (cx <= 1) v = Op::apply(v, dpp<0x121>(v));
+  if (lanes >= 32) {
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                              false);
+    v = Op::apply(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  }
+  if (lanes >= 64) {
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                              false);
+    v = Op::apply(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  }
+  return v;
+}
+
+// All-reduce of the lane's V columns over a unit's lines.  `lds` serves one
+// reduction per kernel (there is no trailing barrier); where a unit has more
+// than one wave every lane of the workgroup must reach the call.
+template <class Op, int V>
+__device__ __forceinline__ void unit_allreduce(float (&v)[V], int cx, int ty_log2,
+                                               float (*lds)[kColMaxLanes * V]) {
+  const int lanes = cx << ty_log2;
+#pragma unroll
+  for (int k = 0; k < V; ++k) v[k] = lines_allreduce<Op>(v[k], cx, lanes);
+  if (lanes <= kWave) return;
+  const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+  const int wave = static_cast<int>(threadIdx.x) >> 6;
+  const int nwaves = lanes >> 6;
+  const int c = lane & (cx - 1);
+  if (lane < cx) {
+#pragma unroll
+    for (int k = 0; k < V; ++k) lds[wave][c * V + k] = v[k];
+  }
+  __syncthreads();
+  const int first = wave & -nwaves;
+#pragma unroll
+  for (int k = 0; k < V; ++k) v[k] = lds[first][c * V + k];
+  for (int w = 1; w < nwaves; ++w)
+#pragma unroll
+    for (int k = 0; k < V; ++k) v[k] = Op::apply(v[k], lds[first + w][c * V + k]);
+}
+
+// Store V columns at p, less the leading ones the vector before this writes.
+template <typename To, int V>
+__device__ __forceinline__ void store_cols(To* __restrict__ p, const float (&o)[V], int shared,
+                                           const Span& s) {
+  if (shared == 0) {
+    store_any<To, V>(p, o, s);
   } else {
-    const float rs = 1.0f / s;
-    for (int r = 0; r < n; ++r) {
-      const float out = fast_exp(xat(r) - m) * rs;
-      store_from_f32<To, 1>(yc + r * inner, &out, sy);
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+      if (k >= shared) store_from_f32<To, 1>(p + k, &o[k], s);
+  }
+}
+
+// The axis in registers: R rows per lane, n <= R << ty_log2, one read and one
+// write of every element; bound by memory.  The kernel it replaced read the
+// axis three times, one element per lane and load.  MI355X, log_softmax over
+// the middle axis, before -> after (the bytes at the copy's rate): fp32
+// 16 x 64 x 16384 57 -> 25.0 us (20.3), bf16 of that size 52 -> 13.2 (10.2),
+// fp16 -> fp32 64 x 512 x 768 469 -> 39 (23), fp32 1 x 4096 x 4096 3780 -> 48
+// (20; 128 bytes of a row per workgroup do not fill the chip, 64 do).
+template <typename Ti, typename To, int V, int R, bool LOG, int B>
+__global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* __restrict__ y,
+                                                  int64_t outer, int n, int64_t inner, int cx,
+                                                  int ty_log2, uint32_t tiles) {
+  typedef typename Raw<Ti, V>::type RT;
+  __shared__ __align__(16) float lds[2][B / kWave][kColMaxLanes * V];
+  const ColLane L = col_lane<V>(outer, inner, cx, ty_log2, tiles);
+  const int rows = L.live && L.ty < n ? ((n - L.ty - 1) >> ty_log2) + 1 : 0;  // the lane's
+  const Span sx = VBH_SPAN(x, outer * n * inner), sy = VBH_SPAN(y, outer * n * inner);
+  const int64_t at = (L.o * n + L.ty) * inner + L.col;
+  const int64_t step = inner << ty_log2;
+  RT xr[R];
+  const RT fill = RT(static_cast<Ti>(kNegInf));
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i < rows) xr[i] = load_any<Ti, V>(x + at + i * step, sx);
+    else xr[i] = fill;
+  }
+  constexpr bool kReload = V * sizeof(Ti) == 16;
+  float m[V], s[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) m[k] = kNegInf;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int k = 0; k < V; ++k) m[k] = max_nan(m[k], raw_at<Ti, V>(xr[i], k));
+  unit_allreduce<Max, V>(m, cx, ty_log2, lds[0]);
+  if constexpr (kReload) reload_barrier<Ti, V, R>(xr);
+#pragma unroll
+  for (int k = 0; k < V; ++k) s[k] = 0.f;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int k = 0; k < V; ++k) s[k] += fast_exp(raw_at<Ti, V>(xr[i], k) - m[k]);
+  unit_allreduce<Sum, V>(s, cx, ty_log2, lds[1]);
+  if constexpr (kReload) reload_barrier<Ti, V, R>(xr);
+#pragma unroll
+  for (int k = 0; k < V; ++k) s[k] = LOG ? fast_log(s[k]) : 1.0f / s[k];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i < rows) {
+      float o[V];
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const float d = raw_at<Ti, V>(xr[i], k) - m[k];
+        o[k] = LOG ? d - s[k] : fast_exp(d) * s[k];
+      }
+      store_cols<To, V>(y + at + i * step, o, L.shared, sy);
+    }
+  }
+}
+
+// Longer axes: an online (max, rescaled sum) pass over the lane's rows, the
+// lines' pairs merged, then an output pass that reads x again.  A column that
+// holds a NaN or +inf, or only -inf, comes out all NaN as torch gives: its max
+// or its sum is NaN, or its max -inf.  fp32 4 x 8192 x 4096: 337 us, 163 at the
+// copy's rate for one read and one write; bf16 of that size 8530 -> 170.
+template <typename Ti, typename To, int V, bool LOG, int B>
+__global__ __launch_bounds__(B) void softmax_cols_stream(const Ti* __restrict__ x,
+                                                         To* __restrict__ y, int64_t outer,
+                                                         int n, int64_t inner, int cx,
+                                                         int ty_log2, uint32_t tiles) {
+  typedef typename Raw<Ti, V>::type RT;
+  constexpr int U = 8;  // rows in flight per lane
+  __shared__ __align__(16) float lds[2][B / kWave][kColMaxLanes * V];
+  const ColLane L = col_lane<V>(outer, inner, cx, ty_log2, tiles);
+  const int rows = L.live && L.ty < n ? ((n - L.ty - 1) >> ty_log2) + 1 : 0;  // the lane's
+  const Span sx = VBH_SPAN(x, outer * n * inner), sy = VBH_SPAN(y, outer * n * inner);
+  const int64_t at = (L.o * n + L.ty) * inner + L.col;
+  const int64_t step = inner << ty_log2;
+  auto load = [&](RT (&v)[U], int i) __attribute__((always_inline)) {
+    const RT fill = RT(static_cast<Ti>(kNegInf));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i + u < rows) v[u] = load_any<Ti, V>(x + at + (i + u) * step, sx);
+      else v[u] = fill;
+    }
+  };
+  float m[V], s[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    m[k] = kNegInf;
+    s[k] = 0.f;
+  }
+  for (int i = 0; i < rows; i += U) {
+    RT v[U];
+    load(v, i);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      float nm = m[k];
+#pragma unroll
+      for (int u = 0; u < U; ++u) nm = max_nan(nm, raw_at<Ti, V>(v[u], k));
+      // all -inf so far: exp(-inf - 0) = 0 instead of NaN
+      const float sh = nm == kNegInf ? 0.f : nm;
+      float e = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u) e += fast_exp(raw_at<Ti, V>(v[u], k) - sh);
+      s[k] = s[k] * fast_exp(m[k] - sh) + e;
+      m[k] = nm;
+    }
+  }
+  float gm[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) gm[k] = m[k];
+  unit_allreduce<Max, V>(gm, cx, ty_log2, lds[0]);
+#pragma unroll
+  for (int k = 0; k < V; ++k)
+    s[k] = m[k] == kNegInf ? 0.f : s[k] * fast_exp(m[k] - gm[k]);
+  unit_allreduce<Sum, V>(s, cx, ty_log2, lds[1]);
+#pragma unroll
+  for (int k = 0; k < V; ++k) s[k] = LOG ? fast_log(s[k]) : 1.0f / s[k];
+  for (int i = 0; i < rows; i += U) {
+    RT v[U];
+    load(v, i);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i + u < rows) {
+        float o[V];
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          const float d = raw_at<Ti, V>(v[u], k) - gm[k];
+          o[k] = LOG ? d - s[k] : fast_exp(d) * s[k];
+        }
+        store_cols<To, V>(y + at + (i + u) * step, o, L.shared, sy);
+      }
     }
   }
 }
@@ -678,21 +849,34 @@ hipError_t launch_softmax_apply(const void* x, void* y, const float* seg_pairs, 
 }
 
 hipError_t launch_softmax_dim(const void* x, void* y, int64_t outer, int n, int64_t inner,
-                              int idt, int odt, int log_mode, hipStream_t s) {
+                              int idt, int odt, int log_mode, const ColGeometry& c,
+                              hipStream_t s) {
   hipError_t err = hipErrorInvalidValue;
-  const int64_t cols = outer * inner;
-  const int block = 256;
-  const int64_t grid = (cols + block - 1) / block;
   dispatch_in_out(idt, odt, [&](auto ti, auto to) {
     using Ti = typename decltype(ti)::type;
     using To = typename decltype(to)::type;
-    if (log_mode)
-      launch_kernel((softmax_mid<Ti, To, true>), dim3(grid), dim3(block), 0, s,
-                         static_cast<const Ti*>(x), static_cast<To*>(y), outer, n, inner);
-    else
-      launch_kernel((softmax_mid<Ti, To, false>), dim3(grid), dim3(block), 0, s,
-                         static_cast<const Ti*>(x), static_cast<To*>(y), outer, n, inner);
-    err = hipGetLastError();
+    auto launch = [&](auto kern) {
+      launch_kernel(kern, dim3(static_cast<uint32_t>(c.grid)), dim3(c.block), 0, s,
+                    static_cast<const Ti*>(x), static_cast<To*>(y), outer, n, inner, c.cx,
+                    c.ty_log2, static_cast<uint32_t>(c.tiles));
+      err = hipGetLastError();
+    };
+    auto go = [&](auto vc, auto lc) {
+      constexpr int V = decltype(vc)::value;
+      constexpr bool LOG = decltype(lc)::value;
+      if (c.rows == 0) launch(softmax_cols_stream<Ti, To, V, LOG, kMaxBlock>);
+      else if (c.rows == 4) launch(softmax_cols<Ti, To, V, 4, LOG, kColBlock>);
+      else if (c.rows == 8 && c.block == kColBlock) launch(softmax_cols<Ti, To, V, 8, LOG, kColBlock>);
+      else if (c.rows == 8) launch(softmax_cols<Ti, To, V, 8, LOG, kMaxBlock>);
+      else if (c.block == kColBlock) launch(softmax_cols<Ti, To, V, 16, LOG, kColBlock>);
+      else launch(softmax_cols<Ti, To, V, 16, LOG, kMaxBlock>);
+    };
+    auto with_log = [&](auto vc) {
+      if (log_mode) go(vc, std::true_type{});
+      else go(vc, std::false_type{});
+    };
+    if (c.v == 1) with_log(std::integral_constant<int, 1>{});
+    else with_log(std::integral_constant<int, Vec<To>::n>{});
   });
   return err;
 }

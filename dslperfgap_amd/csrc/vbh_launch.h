@@ -178,9 +178,27 @@ hipError_t launch_rms_norm(const void* x, const void* w, void* y, int64_t rows,
                            hipStream_t s);
 hipError_t launch_softmax(const void* x, void* y, int64_t rows, int cols, int idt,
                           int odt, int log_mode, const Geometry& g, hipStream_t s);
+// Launch shape of a kernel over column tiles (col_lane in vbh_device.h): `v`
+// elements per lane, `cx` lanes per line of a tile, 2^ty_log2 lines per unit,
+// `tiles` units per outer slab, `grid` workgroups of `block` lanes.  Reductions:
+// the axis cut into `segs` segments of seg_n rows (the last one shorter).
+// Softmax: `rows` of the axis in registers per lane (0: the streaming kernel).
+constexpr int kColBlock = 256;
+constexpr int kColMaxSegs = 64;
+struct ColGeometry {
+  int v = 1;
+  int block = kColBlock;
+  int cx = 1;
+  int ty_log2 = 0;
+  int64_t tiles = 1;
+  int64_t grid = 1;
+  int segs = 1;
+  int seg_n = 0;
+  int rows = 0;
+};
 hipError_t launch_softmax_dim(const void* x, void* y, int64_t outer, int n,
                               int64_t inner, int idt, int odt, int log_mode,
-                              hipStream_t s);
+                              const ColGeometry& c, hipStream_t s);
 // Second stage of a split softmax / log_softmax: y from x and each row's
 // `segs` (<= 64) segment SegPairs (seg_pairs[2 * (row * segs + k)], written by
 // launch_logsumexp_pairs), one kApplyLanes-lane workgroup per tile of
@@ -279,21 +297,6 @@ hipError_t launch_cross_entropy_bwd(const CeBwdArgs& a, hipStream_t s);
 hipError_t launch_reduce(const void* x, void* vals, int64_t* idx, int64_t outer, int n, int idt,
                          int odt, int op, const Geometry& g, hipStream_t s);
 
-// Launch shape of a kernel over column tiles (col_lane in vbh_device.h): `v`
-// elements per lane, `cx` lanes per line of a tile, 2^ty_log2 lines per unit,
-// `tiles` units per outer slab, `grid` workgroups, the axis cut into `segs`
-// segments of seg_n rows (the last one shorter).
-constexpr int kColBlock = 256;
-constexpr int kColMaxSegs = 64;
-struct ColGeometry {
-  int v = 1;
-  int cx = 1;
-  int ty_log2 = 0;
-  int64_t tiles = 1;
-  int64_t grid = 1;
-  int segs = 1;
-  int seg_n = 0;
-};
 // Reduction over the middle axis.  With c.segs > 1, `parts` holds
 // outer * inner * segs fp32 results, and as many int32 rows for max / argmax.
 hipError_t launch_reduce_cols(const void* x, void* vals, int64_t* idx, void* parts,
