@@ -1171,6 +1171,10 @@ int vbh_cross_entropy_fwd_ws(const void* logits, const void* labels, int logits_
         n_cols >= kCePersistMinChunks * cross_entropy_fwd_persist_chunk_cols())))
     return hip_status(launch_cross_entropy_fwd_persist(a, 0, ce_block > 0 ? ce_block : 0, s),
                       "cross_entropy_fwd launch");
+  // longer rows in launches of many: several workgroups per CU walking them
+  if (g_tpr[VBH_OP_CROSS_ENTROPY].load() <= 0 && ce_block <= 0 && !(over & kFlagNoPersist) &&
+      cross_entropy_fwd_any_fits(a))
+    return hip_status(launch_cross_entropy_fwd_any(a, s), "cross_entropy_fwd launch");
   const bool mis_ok = !vec_ok && aligned16(logits) && bs >= kMisMinVecs * vn;
   Geometry g = geometry_for(VBH_OP_CROSS_ENTROPY, bs, vec_ok || mis_ok ? vn : 1, segments, 0,
                             ncb > 1);

@@ -413,28 +413,66 @@ __global__ __launch_bounds__(kMaxBlock) void ce_fwd_stream(
 // Buffer loads with a range of one row: vectors past its end (the last
 // chunk's spare lanes, the loads past a workgroup's last row) read nothing.
 constexpr int kCePersistChunk = 2048;  // 16-byte vectors per chunk (32 KiB)
-constexpr int kCePersistBufs = 2;      // chunks in rotation (loads NB - 1 ahead)
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// acc + the sum of a 16-bit vector's values, two per instruction
+template <typename T, int V>
+__device__ __forceinline__ float add_pairs(const typename Raw<T, V>::type& r, float acc) {
+  if constexpr (sizeof(T) == 2) {
+    typename Pair<T>::type one, x;
+    one[0] = one[1] = static_cast<T>(1.0f);
+#pragma unroll
+    for (int k = 0; k < V; k += 2) {
+      x[0] = r[k];
+      x[1] = r[k + 1];
+      acc = Pair<T>::dot(x, one, acc);
+    }
+  }
+  return acc;
+}
 
-template <int U>
+template <typename T, int U>
 struct CeChunk {
-  f32x4 v[U];
+  typename Raw<T, Vec<T>::n>::type v[U];
 };
+
+// ANY: rows of any length, stride, alignment and type, several workgroups per
+// CU, no barrier inside a row, global loads at 16-byte boundaries (a row's
+// first and last vectors masked).  16-bit rows have twice the exps per byte --
+// about 45 us of VALU work against 56 us of memory time for bf16 4096 x 50257
+// -- so they need waves that fold while others wait for loads: one 512-lane
+// workgroup per CU in step takes 129 us there, four of 256 lanes without the
+// barrier 68 (5.9 chunks of 16 KiB in flight per CU; U = 4 or three buffers
+// 72-90).  Vectors at 16-byte boundaries: off them that launch takes 88.
+// MI355X, ce_fwd_rows (ce_fwd_stream at 128256 columns) -> this: bf16
+// 4096 x 50257 93 -> 69 us, with smoothing 132 -> 74; bf16 4096 x 50304 88 -> 69;
+// fp16 4096 x 40000 98 -> 56; bf16 4096 x 128256 191 -> 163; bf16 512 x 50257
+// 15.0 -> 12.9; fp32 4096 x 50257 163 -> 127 (512-lane workgroups, two per CU),
+// with smoothing 175 -> 127.  Rows of up to kCeAnyMinBytes16 / 32 keep ce_fwd_rows,
+// which holds them in half a workgroup's registers: bf16 8192 x 32000 80
+// against 90 us, fp32 8192 x 32001 154 against 161.
+constexpr int64_t kCeAnyMinRows = 512;
+constexpr int64_t kCeAnyMinBytes16 = int64_t(64) << 10;
+constexpr int64_t kCeAnyMinBytes32 = int64_t(128) << 10;
+// So do aligned 16-bit rows that fill 4 waves of 8 vectors per lane, 8, 12 or
+// 16 of them (bf16 4096 x 65536 84 against 90 us, 1500 x 49152 28.7 against
+// 29.8; but 14 waves, 4096 x 57344, 94 against 79).
+constexpr int64_t kCeAnyFullCols = 16384;
 
 // SL: the row's sum of scaled logits is needed (smoothing); ONE: logit_scale
 // is 1 (else each logit's product with it is rounded once, as the golden
 // rounds it, and used for the max, the exps and the sum).  L: lanes per
-// workgroup (256 or 512), each loading kCePersistChunk / L vectors per chunk.
-template <bool SL, typename LabelT, bool ONE, int L>
+// workgroup, each loading U vectors per chunk, NB chunks in rotation.
+template <typename T, bool SL, typename LabelT, bool ONE, int L, int NB, int U, bool ANY>
 __global__ __launch_bounds__(L) void ce_fwd_persist(
-    const float* __restrict__ logits, const LabelT* __restrict__ labels,
+    const T* __restrict__ logits, const LabelT* __restrict__ labels,
     float* __restrict__ loss, float* __restrict__ lse_out, float* __restrict__ z_out,
     int64_t n_rows, int n_cols, int64_t ld, CeScalars c) {
-  constexpr int CH = kCePersistChunk, U = CH / L;
+  constexpr int CH = U * L;
+  constexpr int V = Vec<T>::n;
+  static_assert(ANY || V == 4, "16-bit rows take global loads");
   constexpr int W = L / kWave;
-  static_assert(U * L == CH && (W & (W - 1)) == 0 && W <= kWave, "a chunk's shape");
-  using Chunk = CeChunk<U>;
+  static_assert((W & (W - 1)) == 0 && W <= kWave, "a chunk's shape");
+  using Chunk = CeChunk<T, U>;
   // per wave, by row parity: the wave's max, its sum of t * exp(m - max) and
   // its sum of logits
   __shared__ float lds_pair[2][3][W];
@@ -443,9 +481,27 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
   const int64_t b = blockIdx.x;
   if (b >= n_rows) return;  // the whole workgroup
   const int64_t grid = gridDim.x;
-  const int nvec = n_cols / 4;
+  // ANY: a row's vectors start at the 16-byte boundary at or before its first
+  // logit, so some rows have one more of them; every row counts the most
+  const int nvec = ANY ? (n_cols + 2 * V - 2) / V : n_cols / V;
   const int cpr = (nvec + CH - 1) / CH;
   const int64_t chunks = ((n_rows - 1 - b) / grid + 1) * cpr;
+  // Where vector j of a row starts, relative to the row: at j * V - lead, moved
+  // into the logits' extent [lo, hi] where the vector would leave it (the first
+  // row's first and the last row's last).
+  struct RowPlace {
+    int lead, lo, hi;
+    __device__ __forceinline__ int at(int j) const { return min(max(j * V - lead, lo), hi); }
+  };
+  auto place = [&](int64_t row) __attribute__((always_inline)) {
+    RowPlace p;
+    const int64_t first = row * ld;
+    p.lead = static_cast<int>((reinterpret_cast<uintptr_t>(logits + first) / sizeof(T)) % V);
+    const int64_t room = strided_extent(n_rows, ld, n_cols) - V - first;
+    p.lo = -static_cast<int>(min(first, int64_t(V)));
+    p.hi = static_cast<int>(min(room, int64_t((nvec - 1) * V - p.lead)));
+    return p;
+  };
   const Span sx = VBH_SPAN(logits, strided_extent(n_rows, ld, n_cols));
   const Span sb = VBH_SPAN(labels, n_rows);
   const Span sloss = VBH_SPAN(loss, n_rows), slse = VBH_SPAN(lse_out, n_rows),
@@ -457,14 +513,23 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
   int lc = 0;
   // (every lambda is inlined: a call would put the captured cursors in memory)
   auto load = [&](Chunk& ch, bool real) __attribute__((always_inline)) {
-    const float* base = logits + (real ? lrow * ld : 0);
-    const bool ok = real && VBH_IN_SPAN(sx, base, static_cast<int64_t>(nvec) * 16);
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(base), static_cast<short>(0), ok ? nvec * 16 : 0, kRawBufferWord3);
+    const T* base = logits + (real ? lrow * ld : 0);
+    if constexpr (ANY) {
+      // loads past the workgroup's last row: the logits' first vector
+      const RowPlace p = place(real ? lrow : 0);
+      const int c0 = real ? lc * CH : 0;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int j = lc * CH + u * L + lane;
-      ch.v[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, j * 16, 0, 2));
+      for (int u = 0; u < U; ++u) ch.v[u] = load_any<T, V>(base + p.at(c0 + u * L + lane), sx);
+    } else {
+      const bool ok = real && VBH_IN_SPAN(sx, base, static_cast<int64_t>(nvec) * 16);
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(base), static_cast<short>(0), ok ? nvec * 16 : 0, kRawBufferWord3);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = lc * CH + u * L + lane;
+        ch.v[u] = __builtin_bit_cast(typename Raw<T, V>::type,
+                                     __builtin_amdgcn_raw_buffer_load_b128(r, j * 16, 0, 2));
+      }
     }
     if (++lc == cpr) {
       lc = 0;
@@ -485,34 +550,62 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
   auto fold_values = [&](const Chunk& ch, auto mask) __attribute__((always_inline)) {
     constexpr bool MASK = decltype(mask)::value;
     const int c0 = fc * CH;
-    float xv[U][4];
+    // MASK: the logits [from, to) of a vector are the lane's -- those of the
+    // row, and not of a vector beside one that was moved; the others count as
+    // -inf, and as 0 in the sum of logits
+    int from[MASK ? U : 1], to[MASK ? U : 1];
+    if constexpr (MASK && ANY) {
+      const RowPlace p = place(frow);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = c0 + u * L + lane, at = p.at(j), nominal = j * V - p.lead;
+        from[u] = max(nominal, 0) - at;
+        to[u] = min(nominal + V, n_cols) - at;
+      }
+    } else if constexpr (MASK) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        from[u] = 0;
+        to[u] = c0 + u * L + lane < nvec ? V : 0;
+      }
+    }
+    auto mine = [&](int u, int k) __attribute__((always_inline)) {
+      return !MASK || (k >= from[MASK ? u : 0] && k < to[MASK ? u : 0]);
+    };
+    // 16-bit rows of scale 1 without a mask take the sum of logits off the raw
+    // pairs, and every 16-bit row widens its logits where they are used
+    constexpr bool WIDE = sizeof(T) == 4 || MASK;
+    float xv[WIDE ? U : 1][V];
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          const float v = raw_at<T, V>(ch.v[u], k);
+          xv[u][k] = mine(u, k) ? (ONE ? v : mul_rn(v, scale)) : kNegInf;
+        }
+    }
+    auto at = [&](int u, int k) __attribute__((always_inline)) {
+      if constexpr (WIDE) return xv[u][k];
+      const float v = raw_at<T, V>(ch.v[u], k);
+      return ONE ? v : mul_rn(v, scale);
+    };
+    float cm = kNegInf;
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) xv[u][k] = ONE ? ch.v[u][k] : mul_rn(ch.v[u][k], scale);
-    float cm = kNegInf;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool ok = !MASK || c0 + u * L + lane < nvec;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) cm = max_nan(cm, ok ? xv[u][k] : kNegInf);
-    }
+      for (int k = 0; k < V; ++k) cm = max_nan(cm, at(u, k));
     const float nm = max_nan(m, cm);
     const float nnb = nm * kLog2e;
-    float xs = 0.f;
     const bool lane_fma = shift_fma_ok(m) && shift_fma_ok(nm);
     if (__builtin_amdgcn_ballot_w64(!lane_fma) == 0) {
       // every lane in the FMA form: s relative to 2^nb
       float e = 0.f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const bool ok = !MASK || c0 + u * L + lane < nvec;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float v = __builtin_amdgcn_exp2f(fmaf(xv[u][k], kLog2e, -nnb));
-          e += ok ? v : 0.f;
-          if constexpr (SL) xs += ok ? xv[u][k] : 0.f;
-        }
+        for (int k = 0; k < V; ++k)
+          e += __builtin_amdgcn_exp2f(fmaf(at(u, k), kLog2e, -nnb));
       }
       // an all -inf share so far holds nothing (its exps would be NaN)
       s = nm == kNegInf ? 0.f : fmaf(s, __builtin_amdgcn_exp2f(nb - nnb), e);
@@ -522,13 +615,8 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
       float e = 0.f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const bool ok = !MASK || c0 + u * L + lane < nvec;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const float v = fast_exp(xv[u][k] - nm);
-          e += ok ? v : 0.f;
-          if constexpr (SL) xs += ok ? xv[u][k] : 0.f;
-        }
+        for (int k = 0; k < V; ++k) e += fast_exp(at(u, k) - nm);
       }
       float t = m == kNegInf ? 0.f
                              : (shift_fma_ok(m) ? s * __builtin_amdgcn_exp2f(-shift_residual(m, nb))
@@ -540,7 +628,19 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
     }
     m = nm;
     nb = nnb;
-    if constexpr (SL) sl += xs;
+    if constexpr (SL) {
+      float xs = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if constexpr (!WIDE && ONE) {
+          xs = add_pairs<T, V>(ch.v[u], xs);
+        } else {
+#pragma unroll
+          for (int k = 0; k < V; ++k) xs += mine(u, k) ? at(u, k) : 0.f;
+        }
+      }
+      sl += xs;
+    }
     // every path has waited for the whole chunk here, so the loads that reuse
     // its registers need no wait of their own
 #pragma unroll
@@ -554,17 +654,19 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
       const int64_t adj = label - c.class_start;
       in_row = adj >= 0 && adj < n_cols;
       logit_raw = 0.f;
-      if (!ignored && in_row && VBH_IN_SPAN(sx, logits + frow * ld + adj, sizeof(float)))
-        logit_raw = logits[frow * ld + adj];
+      if (!ignored && in_row && VBH_IN_SPAN(sx, logits + frow * ld + adj, sizeof(T)))
+        logit_raw = static_cast<float>(logits[frow * ld + adj]);
       const int64_t nrow = frow + grid < n_rows ? frow + grid : n_rows - 1;
       label_next = VBH_IN_SPAN(sb, labels + nrow, sizeof(LabelT)) ? labels[nrow] : LabelT(0);
     }
-    if (fc == cpr - 1) fold_values(ch, std::true_type{});
+    // ANY: a row's last vector is number nvec - 1 or nvec - 2
+    const bool edge = ANY ? fc == 0 || (fc + 1) * CH > nvec - 2 : fc == cpr - 1;
+    if (edge) fold_values(ch, std::true_type{});
     else fold_values(ch, std::false_type{});
     // the waves issue each chunk's loads together: a barrier after every
     // chunk (the row's last one has the merge's) kept them in step, +1% at C4
     // on MI355X against a barrier per row only
-    if (fc != cpr - 1) __syncthreads();
+    if (!ANY && fc != cpr - 1) __syncthreads();
     if (fc == cpr - 1) {
       // each wave merges its lanes' pairs into one (a NaN max or sum
       // propagates into it), one LDS exchange and one barrier per row, and
@@ -611,7 +713,6 @@ __global__ __launch_bounds__(L) void ce_fwd_persist(
     }
   };
 
-  constexpr int NB = kCePersistBufs;
   Chunk buf[NB];
 #pragma unroll
   for (int i = 0; i < NB - 1; ++i) load(buf[i], i < chunks);
@@ -889,7 +990,7 @@ hipError_t launch_cross_entropy_fwd_persist(const CeArgs& a, int64_t max_grid, i
   if (lanes == 0) {
     const int64_t cpr = (a.n_cols / 4 + kCePersistChunk - 1) / kCePersistChunk;
     const int64_t cus = resident_blocks(
-        reinterpret_cast<const void*>(ce_fwd_persist<false, int64_t, true, 256>), 256, 1);
+        reinterpret_cast<const void*>(ce_fwd_persist<float, false, int64_t, true, 256, 2, 8, false>), 256, 1);
     lanes = a.n_rows * cpr >= kCePersistWideChunksPerCu * cus ? 256 : 512;
   }
   hipError_t err = hipErrorInvalidValue;
@@ -904,13 +1005,14 @@ hipError_t launch_cross_entropy_fwd_persist(const CeArgs& a, int64_t max_grid, i
   auto pick = [&](auto lt, auto lc) {
     using LabelT = typename decltype(lt)::type;
     constexpr int L = decltype(lc)::value;
+    constexpr int U = kCePersistChunk / L;
     const LabelT* labels = static_cast<const LabelT*>(a.labels);
     if (c.logit_scale == 1.f) {
-      if (c.has_smoothing) launch(ce_fwd_persist<true, LabelT, true, L>, labels, L);
-      else launch(ce_fwd_persist<false, LabelT, true, L>, labels, L);
+      if (c.has_smoothing) launch(ce_fwd_persist<float, true, LabelT, true, L, 2, U, false>, labels, L);
+      else launch(ce_fwd_persist<float, false, LabelT, true, L, 2, U, false>, labels, L);
     } else {
-      if (c.has_smoothing) launch(ce_fwd_persist<true, LabelT, false, L>, labels, L);
-      else launch(ce_fwd_persist<false, LabelT, false, L>, labels, L);
+      if (c.has_smoothing) launch(ce_fwd_persist<float, true, LabelT, false, L, 2, U, false>, labels, L);
+      else launch(ce_fwd_persist<float, false, LabelT, false, L, 2, U, false>, labels, L);
     }
   };
   auto by_labels = [&](auto lc) {
@@ -919,6 +1021,51 @@ hipError_t launch_cross_entropy_fwd_persist(const CeArgs& a, int64_t max_grid, i
   };
   if (lanes == 256) by_labels(std::integral_constant<int, 256>{});
   else by_labels(std::integral_constant<int, 512>{});
+  return err;
+}
+
+bool cross_entropy_fwd_any_fits(const CeArgs& a) {
+  const bool f32 = a.logits_dt == kF32;
+  if (!f32 && a.n_cols % kCeAnyFullCols == 0 && a.n_cols <= 4 * kCeAnyFullCols &&
+      a.n_rows >= 2 * kCeAnyMinRows && a.ld % 8 == 0 &&
+      (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0)
+    return false;
+  return a.ncb == 1 && a.n_rows >= kCeAnyMinRows && a.n_cols < (1 << 28) &&
+         a.n_cols * (f32 ? 4 : 2) > (f32 ? kCeAnyMinBytes32 : kCeAnyMinBytes16);
+}
+
+hipError_t launch_cross_entropy_fwd_any(const CeArgs& a, hipStream_t s) {
+  const CeScalars c =
+      make_scalars(a.smoothing, a.logit_scale, a.lse_square_scale, a.total_classes,
+                   a.ignored_index, a.class_start, a.has_smoothing, a.split);
+  hipError_t err = hipErrorInvalidValue;
+  dispatch_float_type(a.logits_dt, [&](auto tt) {
+    using T = typename decltype(tt)::type;
+    constexpr int L = sizeof(T) == 4 ? 512 : 256;
+    auto launch = [&](auto kern, auto labels) {
+      const int64_t most = std::max<int64_t>(
+          resident_blocks(reinterpret_cast<const void*>(kern), L, 1024 / L), 1);
+      // as many rows for every workgroup as the busiest one has
+      const int64_t each = (a.n_rows + most - 1) / most;
+      launch_kernel(kern, dim3((a.n_rows + each - 1) / each), dim3(L), 0, s,
+                    static_cast<const T*>(a.logits), labels, a.loss, a.lse, a.z_loss, a.n_rows,
+                    a.n_cols, a.ld, c);
+      err = hipGetLastError();
+    };
+    auto pick = [&](auto lt) {
+      using LabelT = typename decltype(lt)::type;
+      const LabelT* labels = static_cast<const LabelT*>(a.labels);
+      if (c.logit_scale == 1.f) {
+        if (c.has_smoothing) launch(ce_fwd_persist<T, true, LabelT, true, L, 2, 2, true>, labels);
+        else launch(ce_fwd_persist<T, false, LabelT, true, L, 2, 2, true>, labels);
+      } else {
+        if (c.has_smoothing) launch(ce_fwd_persist<T, true, LabelT, false, L, 2, 2, true>, labels);
+        else launch(ce_fwd_persist<T, false, LabelT, false, L, 2, 2, true>, labels);
+      }
+    };
+    if (a.label_i64) pick(TypeTag<int64_t>{});
+    else pick(TypeTag<int32_t>{});
+  });
   return err;
 }
 

@@ -63,23 +63,6 @@ __device__ __forceinline__ float tree_sum(const float (&a)[V]) {
   return t[0];
 }
 
-// Products of 16-bit pairs on the packed dot-product unit: a.lo * b.lo +
-// a.hi * b.hi + c (v_dot2c_f32_bf16 / v_dot2c_f32_f16; the products of 16-bit
-// values are exact in fp32), two values per instruction and no widening.
-template <typename T> struct Pair;
-template <> struct Pair<__bf16> {
-  typedef __bf16 type __attribute__((ext_vector_type(2)));
-  __device__ static float dot(type a, type b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(a, b, c, false);
-  }
-};
-template <> struct Pair<_Float16> {
-  typedef _Float16 type __attribute__((ext_vector_type(2)));
-  __device__ static float dot(type a, type b, float c) {
-    return __builtin_amdgcn_fdot2(a, b, c, false);
-  }
-};
-
 // sum over the lane's 16-bit values of x * (SQ ? x : 1), V / 2 accumulators
 template <typename T, int V, int IT, bool SQ>
 __device__ __forceinline__ float lane_dot2_sum(const typename Raw<T, V>::type (&xr)[IT]) {

@@ -258,6 +258,11 @@ bool cross_entropy_fwd_persist_fits(int logits_dtype, int64_t n_cols);
 int64_t cross_entropy_fwd_persist_chunk_cols();
 hipError_t launch_cross_entropy_fwd_persist(const CeArgs& a, int64_t max_grid, int lanes,
                                             hipStream_t s);
+// The forward for long rows of any length, stride, alignment and type in
+// launches of many rows (ce_fwd_persist, ANY): whether it is the faster one for
+// `a`, and its launch.
+bool cross_entropy_fwd_any_fits(const CeArgs& a);
+hipError_t launch_cross_entropy_fwd_any(const CeArgs& a, hipStream_t s);
 // Second stage of a split row: `a` describes the caller's launch (one column
 // block per row); seg_loss / seg_lse hold the first stage's `segs` segments
 // per row at flat index k * n_rows + row.

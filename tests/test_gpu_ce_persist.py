@@ -6,9 +6,11 @@ workgroup per CU folding its rows chunk by chunk into per-lane online (max,
 sum of exp) pairs, in workgroups of 256 lanes from 64 chunks per CU up and of
 512 below; the tune flag TUNE_PERSIST takes it down to one chunk (8192
 columns) and any row count, and with a block override of 256 or 512 sets the
-workgroup size (both are run on every case here).  16-bit logits and column
-blocks stay on
-ce_fwd_rows (cases below as well).  These tests hold it to the oracle (the restated
+workgroup size (both are run on every case here).  Launches of 512 rows or more
+of 64 KiB (16-bit) or 128 KiB (fp32) that the above leaves take its other form,
+which reads rows of any length, stride, alignment and type from the 16-byte
+boundary before them; shorter 16-bit rows and column blocks stay on ce_fwd_rows
+(cases below as well).  These tests hold it to the oracle (the restated
 golden, oracle/pytorch_impl.py) at the strict fp32 tolerance of the measured
 configs, on every output, with the golden's special values (NaN, +inf, all
 -inf rows, -inf chunks inside finite rows, rows at +-FLT_MAX), shifted labels,
@@ -211,3 +213,31 @@ def test_persistent_cross_entropy_strided_rows(rows, cols, pad):
         _lib.tune_override(_lib.OP_CROSS_ENTROPY, 0, 0, 0)
     want = ref.cross_entropy_fwd(logits, labels, *args)
     _check(got, want, rows, f"strided {rows}x{cols} pad {pad}")
+
+
+# the form for any row: lengths around whole vectors and chunks (a chunk is 512
+# 16-bit or 1024 fp32 vectors; at 36858-36865 16-bit and 36862-36865 fp32
+# columns a row's vectors number one more than whole chunks), odd strides, and
+# buffers that start off a 16-byte boundary
+ANY_CASES = [(torch.bfloat16, 512, 32769, 0, 0), (torch.float16, 513, 32776, 0, 0),
+             (torch.bfloat16, 1030, 36859, 0, 0), (torch.bfloat16, 520, 36864, 3, 5),
+             (torch.float16, 530, 36865, 0, 1), (torch.bfloat16, 600, 66003, 8, 0),
+             (torch.float32, 512, 32772, 0, 0), (torch.float32, 540, 36863, 0, 3),
+             (torch.float32, 520, 36865, 6, 0), (torch.float32, 515, 65601, 0, 2)]
+
+
+@pytest.mark.parametrize("dtype,rows,cols,pad,offset", ANY_CASES)
+@pytest.mark.parametrize("pi", [0, 1, 3])
+def test_any_row_cross_entropy_matches_oracle(dtype, rows, cols, pad, offset, pi):
+    start = cols // 7
+    logits, labels = _inputs(rows, cols, dtype, 960 + rows + pi, start)
+    store = torch.full((offset + rows * (cols + pad),), float("nan"), dtype=dtype, device=DEV)
+    xd = store[offset:].view(rows, cols + pad)[:, :cols]
+    xd.copy_(logits)  # the gaps between rows hold NaN
+    labels = labels.to(torch.int32) if pi == 1 else labels
+    args = dict(ignored_index=-100, total_classes=cols + start, class_start_idx=start,
+                BLOCK_SIZE=cols, **PARAMS[pi])
+    print(f"[ce persist] any {rows}x{cols} {dtype} pad={pad} offset={offset} params {pi}",
+          flush=True)
+    got = cross_entropy_fwd(xd, labels.to(DEV), **args)
+    _check(got, ref.cross_entropy_fwd(logits, labels, **args), rows, f"any {rows}x{cols} {dtype}")
