@@ -99,16 +99,18 @@ constexpr int64_t kShortRowVecs = 32;
 constexpr int kItShort[kNumOps] = {2, 2, 2, 2, 4, 4};
 constexpr int kMinLanesShort[kNumOps] = {4, 8, 8, 8, 2, 4};
 
-int it_target(int op, int64_t nvec, int vec, bool column_blocks) {
+int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in) {
   if (vec > 1 && nvec <= kShortRowVecs) {
     int it = kItShort[op];
     while (it > 1 && nvec / it < kMinLanesShort[op]) it /= 2;
     return it;
   }
-  // fp32 softmax rows of 33-64 vectors: one wave per row (log_softmax fp32,
+  // softmax rows of 33-64 vectors: one wave per row of fp32 (log_softmax fp32,
   // 64 MB per call: 256 columns 5730 -> 5849 GB/s, 255 columns 4843 -> 5241;
-  // 512 columns and more keep 2 vectors per lane, within 1% of the best)
-  if (op == VBH_OP_SOFTMAX && vec == 4 && nvec <= kWave) return 1;
+  // 512 columns and more keep 2 vectors per lane, within 1% of the best), 4 of
+  // the 8-byte vectors of 16-bit rows written as fp32 (bf16 20000 x 255 at 1 / 2
+  // / 4 vectors 9.6 / 9.0 / 7.3 us, fp16 50000 x 135 17.2 / 12.8 / 12.7)
+  if (op == VBH_OP_SOFTMAX && vec == 4 && nvec <= kWave) return half_in ? 4 : 1;
   // 16-bit LayerNorm rows of 1025-1536 vectors: 2 vectors per lane, 9-12 waves
   // per row (bf16 at 64 MB per call, 4 -> 2: 9216 columns 4298 -> 5247 GB/s,
   // 10240 4501 -> 5194, 11264 4855 -> 5199, 12288 5126 -> 5290; at 768 and
@@ -327,8 +329,9 @@ Geometry geometry_for(int op, int64_t cols, int vec, int64_t units, int64_t out_
   const bool norm = op == VBH_OP_LAYER_NORM || op == VBH_OP_RMS_NORM;
   if (norm && !(over & kFlagNoPersist)) flags |= kFlagPersist;
   const int64_t nvec = cols / vec;
+  const bool half_in = dtype == kF16 || dtype == kBF16;
   Geometry g =
-      pick_geometry(cols, vec, fill_it(it_target(op, nvec, vec, column_blocks), nvec, units),
+      pick_geometry(cols, vec, fill_it(it_target(op, nvec, vec, column_blocks, half_in), nvec, units),
                     g_tpr[op].load(), g_block[op].load(), flags);
   if (g.persist && !(over & kFlagPersist) && g.tpr < kPersistMinTpr[op]) g.persist = false;
   // LayerNorm row groups of exactly 2 waves run 4 to a 512-lane workgroup
@@ -418,7 +421,7 @@ Geometry reduce_geometry(int64_t n, int vec, int64_t units) {
   const int64_t nvec = n / vec;
   int tpr = g_tpr[VBH_OP_REDUCE].load();
   if (tpr <= 0) {
-    const int per_lane = fill_it(it_target(VBH_OP_REDUCE, nvec, vec, false), nvec, units);
+    const int per_lane = fill_it(it_target(VBH_OP_REDUCE, nvec, vec, false, false), nvec, units);
     const int64_t lanes = (nvec + per_lane - 1) / per_lane;
     if (lanes <= kWave) {
       tpr = pow2ceil(lanes < 1 ? 1 : lanes);
@@ -926,13 +929,14 @@ int vbh_softmax_fwd_ws(const void* x, void* y, int64_t rows, int64_t cols, int i
   if (rows == 0 || cols == 0) return 0;
   if (!x || !y) return fail(VBH_E_INVALID, "softmax: null pointer");
   const int vn = 16 / elt_size(in_dtype);
+  const int vo = std::min(vn, 16 / elt_size(out_dtype));  // of the kernels that write y
   const bool aligned = aligned16(x) && aligned16(y);
-  const bool vec_ok = cols % vn == 0 && aligned;
-  const bool mis_ok = !vec_ok && aligned && cols >= kMisMinVecs * vn;
+  const bool vec_ok = cols % vo == 0 && aligned;
+  const bool mis_ok = !vec_ok && aligned && cols >= kMisMinVecs * vo;
   const int64_t out_bytes = mul_sat(mul_sat(rows, cols), elt_size(out_dtype));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t need = vbh_softmax_workspace_bytes(rows, cols, in_dtype);
-  if (need > 0 && (vec_ok || mis_ok) && workspace != nullptr && workspace_bytes >= need &&
+  if (need > 0 && aligned && workspace != nullptr && workspace_bytes >= need &&
       aligned16(workspace)) {
     // segment SegPairs (fp32 max, sum of exp): the [rows * segs, cols / segs]
     // view, or the MIS kernel's segment mode; then one pass over x that
@@ -942,23 +946,25 @@ int vbh_softmax_fwd_ws(const void* x, void* y, int64_t rows, int64_t cols, int i
     const int64_t units = rows * segs;
     const int seg_cols = static_cast<int>(sp.seg_cols);
     Geometry g1 = geometry_for(VBH_OP_LOGSUMEXP, seg_cols, vn, units);
-    Geometry g2 = geometry_for(VBH_OP_SOFTMAX, cols, vn, rows, out_bytes);  // nt / wt
+    Geometry g2 = geometry_for(VBH_OP_SOFTMAX, cols, vo, rows, out_bytes);  // nt / wt
     g2.mis = !vec_ok;
-    if (vec_ok || use_mis(g1, vn)) {
+    const bool even = cols % vn == 0;
+    if (even || use_mis(g1, vn)) {
       if (int rc = check_grid(units, g1)) return rc;
       float* seg_pairs = static_cast<float*>(workspace);
       hipError_t e =
-          vec_ok ? launch_logsumexp_pairs(x, seg_pairs, units, seg_cols, in_dtype, g1, s)
-                 : launch_logsumexp_pairs(x, seg_pairs, units, static_cast<int>(cols), in_dtype,
-                                          g1, s, segs, seg_cols);
+          even ? launch_logsumexp_pairs(x, seg_pairs, units, seg_cols, in_dtype, g1, s)
+               : launch_logsumexp_pairs(x, seg_pairs, units, static_cast<int>(cols), in_dtype, g1,
+                                        s, segs, seg_cols);
       if (e == hipSuccess)
         e = launch_softmax_apply(x, y, seg_pairs, rows, static_cast<int>(cols), segs, in_dtype,
                                  out_dtype, log_mode, g2, s);
       return hip_status(e, "softmax launch");
     }
   }
-  Geometry g = geometry_for(VBH_OP_SOFTMAX, cols, vec_ok || mis_ok ? vn : 1, rows, out_bytes);
-  if (mis_ok && !use_mis(g, vn)) g = geometry_for(VBH_OP_SOFTMAX, cols, 1, rows, out_bytes);
+  Geometry g = geometry_for(VBH_OP_SOFTMAX, cols, vec_ok || mis_ok ? vo : 1, rows, out_bytes, false,
+                            in_dtype);
+  if (mis_ok && !use_mis(g, vo)) g = geometry_for(VBH_OP_SOFTMAX, cols, 1, rows, out_bytes);
   if (int rc = check_grid(rows, g)) return rc;
   return hip_status(launch_softmax(x, y, rows, static_cast<int>(cols), in_dtype, out_dtype,
                                    log_mode, g, s),

@@ -111,6 +111,29 @@ __device__ __forceinline__ MisRow mis_row(int64_t start, int cols) {
   return MisRow{head, nvec, cols - head - nvec * V};
 }
 
+// Elements per lane access of a softmax: 16 bytes of the wider type.  16-bit
+// rows written as fp32 load 8 bytes per lane, so that the lanes' 16-byte stores
+// lie side by side; with 8 elements per lane every store left 16-byte gaps for
+// the next one (MI355X, bf16 -> fp32
+// log_softmax, 8 -> 4 elements: 1024 x 50257 91 -> 71 us, 8192 x 4096 52.6 -> 33.5,
+// 512 x 65536 68 -> 40).
+template <typename Ti, typename To>
+constexpr int softmax_vec = Vec<To>::n < Vec<Ti>::n ? Vec<To>::n : Vec<Ti>::n;
+
+// The row's exp form for softmax of fp32 rows of 64 values per lane: both forms
+// of ExpFma and ExpSub in one, 2^((x - m1) * log2 e - mb) with m1 = 0 or mb = 0,
+// for a subtract per element.  With the two forms beside each other the
+// kernel's 128 VGPRs did not hold the row (42-59 of them spilled).  MI355X,
+// softmax fp32 1000 x 65536 130 -> 104 us, 2048 x 50257 191 -> 167.
+struct ExpEither {
+  float m1, mb;
+  __device__ __forceinline__ float operator()(float x) const {
+    return __builtin_amdgcn_exp2f(fmaf(x - m1, kLog2e, -mb));
+  }
+};
+template <typename Ti, int V, int IT, bool LOG>
+constexpr bool kOneExpForm = !LOG && sizeof(Ti) == 4 && V * IT >= 64;
+
 template <typename Ti, typename To, int V, int IT, bool LOG, int SP, bool MIS>
 __global__ __launch_bounds__(kMaxBlock) void softmax_rows(const Ti* __restrict__ x,
                                                           To* __restrict__ y, int64_t rows,
@@ -147,8 +170,12 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_rows(const Ti* __restrict__
   const float mb = m * kLog2e;
   const ExpFma efma{mb};
   const ExpSub esub{m};
-  float le = fma_ok ? lane_sum_exp<Ti, V, IT, KEEP>(xr, efma)
-                    : lane_sum_exp<Ti, V, IT, KEEP>(xr, esub);
+  float le;
+  if constexpr (kOneExpForm<Ti, V, IT, LOG>)
+    le = lane_sum_exp<Ti, V, IT, KEEP>(xr, ExpEither{fma_ok ? 0.f : m, fma_ok ? mb : 0.f});
+  else
+    le = fma_ok ? lane_sum_exp<Ti, V, IT, KEEP>(xr, efma)
+                : lane_sum_exp<Ti, V, IT, KEEP>(xr, esub);
   if (hv) le += fma_ok ? efma(hx) : esub(hx);
   if (tv) le += fma_ok ? efma(tx) : esub(tx);
   const float s = group_allreduce<Sum>(le, tpr, lds[1]);
@@ -373,78 +400,84 @@ __global__ __launch_bounds__(kApplyLanes) void softmax_apply_tiles(
 // streaming (one workgroup per row)
 // ---------------------------------------------------------------------------
 
-// Online row statistics for the streaming path: running max `m` (NaN ignored),
-// sum `s` of exp(x - m) rescaled whenever m grows, and a NaN flag.  The final
+// Online row statistics for the streaming path: running max `m` (NaN if a
+// value is NaN), and sum `s` of exp(x - m) rescaled whenever m grows, kStreamU
+// vectors per lane in flight.  s is meaningless where m is NaN or infinite; the
 // outputs reproduce torch's special values explicitly:
 //   softmax / log_softmax: a row holding NaN or +inf, or only -inf, is all NaN;
 //   logsumexp: NaN row -> NaN, a +inf max -> +inf, an all -inf row -> -inf.
 struct RowStats {
-  float m, s, nan;
+  float m, s;
+  __device__ __forceinline__ bool special() const { return m != m || __builtin_isinf(m); }
 };
 
-template <typename T, int V>
+// The first pass leaves the row in the caches for the second (nontemporal
+// loads there cost bf16 300 x 131072 53 us against 42).  MI355X, one vector in
+// flight -> four: logsumexp fp32 600 x 100000 55 -> 39.5 us, softmax fp32
+// 900 x 131072 268 -> 215, log_softmax fp16 -> fp32 300 x 131072 79 -> 54.
+constexpr int kStreamU = 4;
+
+template <typename T, int V, bool NT>
+__device__ __forceinline__ void stream_load(const T* __restrict__ xr, int j0, int nvec,
+                                            typename Raw<T, V>::type (&v)[kStreamU],
+                                            const Span& sx) {
+  const typename Raw<T, V>::type fill = typename Raw<T, V>::type(static_cast<T>(kNegInf));
+#pragma unroll
+  for (int u = 0; u < kStreamU; ++u) {
+    const int j = j0 + u * kMaxBlock;
+    if (j < nvec) v[u] = load_raw<T, V, NT>(xr + static_cast<int64_t>(j) * V, sx);
+    else v[u] = fill;
+  }
+}
+
+// (the streaming kernels run kMaxBlock lanes per row)
+template <typename T, int V, bool NT>
 __device__ __forceinline__ RowStats stream_stats(const T* __restrict__ xr, int nvec,
                                                  float* lds, const Span& sx) {
-  float m = kNegInf, s = 0.f, nan = 0.f;
-  for (int j = threadIdx.x; j < nvec; j += blockDim.x) {
-    float v[V];
-    load_f32<T, V>(xr + static_cast<int64_t>(j) * V, v, sx);
-    float cm = kNegInf;
-#pragma unroll
-    for (int k = 0; k < V; ++k) {
-      cm = fmaxf(cm, v[k]);
-      if (v[k] != v[k]) nan = 1.f;
-    }
-    if (cm > m) {
-      s = (m == kNegInf) ? 0.f : s * fast_exp(m - cm);
-      m = cm;
-    }
-    if (m != kNegInf && m != -kNegInf) {
-#pragma unroll
-      for (int k = 0; k < V; ++k) s += (v[k] != v[k]) ? 0.f : fast_exp(v[k] - m);
-    }
+  float m = kNegInf, s = 0.f;
+  for (int j = threadIdx.x; j < nvec; j += kStreamU * kMaxBlock) {
+    typename Raw<T, V>::type v[kStreamU];
+    stream_load<T, V, NT>(xr, j, nvec, v, sx);
+    const float nm = max_nan(m, lane_max<T, V, kStreamU>(v));
+    const float sh = nm == kNegInf ? 0.f : nm;  // exp(-inf - 0) = 0 instead of NaN
+    s = s * fast_exp(m - sh) + lane_sum_exp<T, V, kStreamU>(v, ExpSub{sh});
+    m = nm;
   }
-  const int tpr = blockDim.x;
-  const float gm = group_allreduce<Max>(m, tpr, lds);
-  const bool finite = gm != kNegInf && gm != -kNegInf;
-  const float t = (finite && m != kNegInf) ? s * fast_exp(m - gm) : 0.f;
-  const float gs = group_allreduce<Sum>(t, tpr, lds + kMaxWaves);
-  const float gn = group_allreduce<Max>(nan, tpr, lds + 2 * kMaxWaves);
-  return RowStats{gm, gs, gn};
+  const float gm = group_allreduce<Max>(m, kMaxBlock, lds);
+  const float t = m == kNegInf ? 0.f : s * fast_exp(m - gm);
+  const float gs = group_allreduce<Sum>(t, kMaxBlock, lds + kMaxWaves);
+  return RowStats{gm, gs};
 }
 
 template <typename Ti, typename To, int V, bool LOG>
 __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const Ti* __restrict__ x,
                                                             To* __restrict__ y, int cols) {
-  __shared__ float lds[3 * kMaxWaves];
+  __shared__ float lds[2 * kMaxWaves];
   const int nvec = cols / V;
   const int64_t row = blockIdx.x;
   const Ti* xr = x + row * cols;
   // one workgroup per row: the grid is the row count
   const Span sx = VBH_SPAN(x, static_cast<int64_t>(gridDim.x) * cols);
   const Span sy = VBH_SPAN(y, static_cast<int64_t>(gridDim.x) * cols);
-  const RowStats st = stream_stats<Ti, V>(xr, nvec, lds, sx);
-  const bool special = st.nan != 0.f || st.m == kNegInf || st.m == -kNegInf;
-  const float qnan = __builtin_nanf("");
+  const RowStats st = stream_stats<Ti, V, false>(xr, nvec, lds, sx);
   const float m = st.m;
+  const float ls = st.special() ? __builtin_nanf("") : (LOG ? fast_log(st.s) : 1.0f / st.s);
   To* yr = y + row * cols;
-  if constexpr (LOG) {
-    const float ls = special ? qnan : fast_log(st.s);
-    for (int j = threadIdx.x; j < nvec; j += blockDim.x) {
-      float v[V], o[V];
-      load_f32<Ti, V>(xr + static_cast<int64_t>(j) * V, v, sx);
+  for (int j0 = threadIdx.x; j0 < nvec; j0 += kStreamU * kMaxBlock) {
+    typename Raw<Ti, V>::type v[kStreamU];
+    stream_load<Ti, V, true>(xr, j0, nvec, v, sx);
 #pragma unroll
-      for (int k = 0; k < V; ++k) o[k] = (v[k] - m) - ls;
-      store_from_f32<To, V>(yr + static_cast<int64_t>(j) * V, o, sy);
-    }
-  } else {
-    const float r = special ? qnan : 1.0f / st.s;
-    for (int j = threadIdx.x; j < nvec; j += blockDim.x) {
-      float v[V], o[V];
-      load_f32<Ti, V>(xr + static_cast<int64_t>(j) * V, v, sx);
+    for (int u = 0; u < kStreamU; ++u) {
+      const int j = j0 + u * kMaxBlock;
+      if (j < nvec) {
+        float o[V];
 #pragma unroll
-      for (int k = 0; k < V; ++k) o[k] = fast_exp(v[k] - m) * r;
-      store_from_f32<To, V>(yr + static_cast<int64_t>(j) * V, o, sy);
+        for (int k = 0; k < V; ++k) {
+          const float d = raw_at<Ti, V>(v[u], k) - m;
+          o[k] = LOG ? d - ls : fast_exp(d) * ls;
+        }
+        store_raw<To, V, true>(yr + static_cast<int64_t>(j) * V, o, sy);
+      }
     }
   }
 }
@@ -453,23 +486,19 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const Ti* __restrict
 template <typename Ti, typename To, int V, bool PAIR = false>
 __global__ __launch_bounds__(kMaxBlock) void logsumexp_stream(const Ti* __restrict__ x,
                                                               To* __restrict__ y, int cols) {
-  __shared__ float lds[3 * kMaxWaves];
+  __shared__ float lds[2 * kMaxWaves];
   const int nvec = cols / V;
   const int64_t row = blockIdx.x;
   // one workgroup per row: the grid is the row count
   const Span sx = VBH_SPAN(x, static_cast<int64_t>(gridDim.x) * cols);
   const Span sy = VBH_SPAN(y, static_cast<int64_t>(gridDim.x) * (PAIR ? 2 : 1));
-  const RowStats st = stream_stats<Ti, V>(x + row * cols, nvec, lds, sx);
+  const RowStats st = stream_stats<Ti, V, true>(x + row * cols, nvec, lds, sx);
   if (threadIdx.x == 0) {
-    const bool inf = st.m == kNegInf || st.m == -kNegInf;
     if constexpr (PAIR) {
-      const float pair[2] = {st.nan != 0.f ? __builtin_nanf("") : st.m, inf ? 0.f : st.s};
+      const float pair[2] = {st.m, __builtin_isinf(st.m) ? 0.f : st.s};
       store_from_f32<float, 2>(reinterpret_cast<float*>(y) + 2 * row, pair, sy);
     } else {
-      float r;
-      if (st.nan != 0.f) r = __builtin_nanf("");
-      else if (inf) r = st.m;
-      else r = fast_log(st.s) + st.m;
+      const float r = st.special() ? st.m : fast_log(st.s) + st.m;
       store_from_f32<To, 1>(y + row, &r, sy);
     }
   }
@@ -573,7 +602,6 @@ __global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* 
     if (i < rows) xr[i] = load_any<Ti, V>(x + at + i * step, sx);
     else xr[i] = fill;
   }
-  constexpr bool kReload = V * sizeof(Ti) == 16;
   float m[V], s[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) m[k] = kNegInf;
@@ -582,7 +610,7 @@ __global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* 
 #pragma unroll
     for (int k = 0; k < V; ++k) m[k] = max_nan(m[k], raw_at<Ti, V>(xr[i], k));
   unit_allreduce<Max, V>(m, cx, ty_log2, lds[0]);
-  if constexpr (kReload) reload_barrier<Ti, V, R>(xr);
+  reload_barrier<Ti, V, R>(xr);
 #pragma unroll
   for (int k = 0; k < V; ++k) s[k] = 0.f;
 #pragma unroll
@@ -590,7 +618,7 @@ __global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* 
 #pragma unroll
     for (int k = 0; k < V; ++k) s[k] += fast_exp(raw_at<Ti, V>(xr[i], k) - m[k]);
   unit_allreduce<Sum, V>(s, cx, ty_log2, lds[1]);
-  if constexpr (kReload) reload_barrier<Ti, V, R>(xr);
+  reload_barrier<Ti, V, R>(xr);
 #pragma unroll
   for (int k = 0; k < V; ++k) s[k] = LOG ? fast_log(s[k]) : 1.0f / s[k];
 #pragma unroll
@@ -704,7 +732,7 @@ hipError_t launch_softmax(const void* x, void* y, int64_t rows, int cols, int id
   dispatch_in_out(idt, odt, [&](auto ti, auto to) {
     using Ti = typename decltype(ti)::type;
     using To = typename decltype(to)::type;
-    constexpr int VN = Vec<Ti>::n;
+    constexpr int VN = softmax_vec<Ti, To>;
     auto go = [&](auto vc, auto lc) {
       constexpr int V = decltype(vc)::value;
       constexpr bool LOG = decltype(lc)::value;
@@ -826,7 +854,7 @@ hipError_t launch_softmax_apply(const void* x, void* y, const float* seg_pairs, 
   dispatch_in_out(idt, odt, [&](auto ti, auto to) {
     using Ti = typename decltype(ti)::type;
     using To = typename decltype(to)::type;
-    constexpr int V = Vec<Ti>::n;
+    constexpr int V = softmax_vec<Ti, To>;
     const int64_t tiles = (cols / V + kApplyLanes - 1) / kApplyLanes;
     dispatch_store_policy<V>(g, [&](auto sp) {
       constexpr int SP = decltype(sp)::value;

@@ -159,11 +159,11 @@ __device__ __forceinline__ float raw_at(const typename Raw<T, V>::type& r, int k
 template <typename T, int V, int IT>
 __device__ __forceinline__ void reload_barrier(typename Raw<T, V>::type (&r)[IT]) {
   if constexpr (sizeof(T) == 2 && V > 1) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    static_assert(sizeof(typename Raw<T, V>::type) == 16, "16-byte vectors expected");
+    typedef uint32_t words __attribute__((ext_vector_type(V / 2)));
+    static_assert(sizeof(typename Raw<T, V>::type) == sizeof(words), "whole words expected");
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-      u32x4 u = __builtin_bit_cast(u32x4, r[i]);
+      words u = __builtin_bit_cast(words, r[i]);
       asm volatile("" : "+v"(u));
       r[i] = __builtin_bit_cast(typename Raw<T, V>::type, u);
     }
