@@ -49,11 +49,62 @@ def _logits(logits, what):
     return logits
 
 
+_raw_device, _raw_stream = _bridge._raw_device, _bridge._raw_stream
+# (logits shape, dtype, labels shape, dtype, BLOCK_SIZE) -> (rows, columns, logits
+# code, label code, entry point), or False where a call needs the general path
+# (which raises the errors of invalid calls)
+_FWD_PLANS = _bridge.PlanCache()
+_BWD_PLANS = _bridge.PlanCache()
+
+
+def _shape_plan(shape, dtype, lshape, ldtype, block):
+    code, lcode = _bridge.FLOAT_CODES.get(dtype), _bridge.LABEL_CODES.get(ldtype)
+    if (code is None or lcode is None or len(shape) != 2 or len(lshape) != 1 or
+            lshape[0] != shape[0] or block <= 0):
+        return False
+    return (int(shape[0]), int(shape[1]), code, lcode)
+
+
+def _fwd_plan(shape, dtype, lshape, ldtype, block):
+    p = _shape_plan(shape, dtype, lshape, ldtype, block)
+    if not p or _lib.cross_entropy_workspace_bytes(p[0], p[1], block, p[2]):
+        return False
+    return (*p, _lib.entry("vbh_cross_entropy_fwd"))
+
+
+def _bwd_plan(shape, dtype, lshape, ldtype, block):
+    p = _shape_plan(shape, dtype, lshape, ldtype, block)
+    return (*p, _lib.entry("vbh_cross_entropy_bwd")) if p else False
+
+
 def cross_entropy_fwd(
     logits, labels, smoothing, logit_scale, lse_square_scale,
     ignored_index, total_classes, class_start_idx, BLOCK_SIZE, HAS_SMOOTHING, SPLIT
 ):
     """Column-blocked CE forward; see the module docstring for the layout."""
+    # the common call: contiguous logits and labels on the current GPU, rows not
+    # split -- one pass over the tensors' attributes, a cached plan per shape
+    if type(BLOCK_SIZE) is int:
+        key = (logits.shape, logits.dtype, labels.shape, labels.dtype, BLOCK_SIZE)
+        p = _FWD_PLANS.get(key)
+        if p is None:
+            p = _FWD_PLANS.put(key, _fwd_plan(*key))
+        if p:
+            dev = logits.get_device()
+            if (dev >= 0 and dev == _raw_device() and labels.get_device() == dev and
+                    logits.is_contiguous() and labels.is_contiguous()):
+                n_rows, n_cols, code, lcode, fn = p
+                loss = torch.empty_like(logits, dtype=torch.float32)
+                lse = torch.empty_like(loss)
+                z_loss = torch.empty_like(loss)
+                rc = fn(logits.data_ptr(), labels.data_ptr(), code, lcode, loss.data_ptr(),
+                        lse.data_ptr(), z_loss.data_ptr(), n_rows, n_cols, n_cols,
+                        float(smoothing), float(logit_scale), float(lse_square_scale),
+                        int(ignored_index), int(total_classes), int(class_start_idx), BLOCK_SIZE,
+                        int(bool(HAS_SMOOTHING)), int(bool(SPLIT)), _raw_stream(dev))
+                if rc != 0:
+                    raise _lib.VbhError("vbh_cross_entropy_fwd", rc, _lib.last_error())
+                return loss, lse, z_loss
     what = "cross_entropy_fwd"
     dev = _bridge.require_gpu(what, logits, labels)
     if int(BLOCK_SIZE) <= 0:
@@ -85,6 +136,29 @@ def cross_entropy_bwd(
     ignored_index, total_classes, class_start_idx, BLOCK_SIZE, HAS_SMOOTHING
 ):
     """dlogits = dloss * logit_scale * (softmax(+ z-loss term) - smoothed one-hot)."""
+    # the common call: contiguous tensors on the current GPU, fp32 dloss and lse
+    if type(BLOCK_SIZE) is int and dloss.dtype is torch.float32 and lse.dtype is torch.float32:
+        key = (logits.shape, logits.dtype, labels.shape, labels.dtype, BLOCK_SIZE)
+        p = _BWD_PLANS.get(key)
+        if p is None:
+            p = _BWD_PLANS.put(key, _bwd_plan(*key))
+        if p:
+            dev = logits.get_device()
+            n_rows, n_cols, code, lcode, fn = p
+            if (dev >= 0 and dev == _raw_device() and labels.get_device() == dev and
+                    dloss.get_device() == dev and lse.get_device() == dev and
+                    logits.is_contiguous() and labels.is_contiguous() and
+                    dloss.is_contiguous() and lse.is_contiguous() and
+                    dloss.numel() >= n_rows and lse.numel() >= n_rows):
+                dlogits = torch.empty_like(logits)
+                rc = fn(dloss.data_ptr(), logits.data_ptr(), lse.data_ptr(), labels.data_ptr(),
+                        dlogits.data_ptr(), code, lcode, n_rows, n_cols, n_cols, n_cols, 1,
+                        float(smoothing), float(logit_scale), float(lse_square_scale),
+                        int(ignored_index), int(total_classes), int(class_start_idx),
+                        int(bool(HAS_SMOOTHING)), _raw_stream(dev))
+                if rc != 0:
+                    raise _lib.VbhError("vbh_cross_entropy_bwd", rc, _lib.last_error())
+                return dlogits
     what = "cross_entropy_bwd"
     dev = _bridge.require_gpu(what, dloss, logits, lse, labels)
     if int(BLOCK_SIZE) <= 0:
@@ -120,6 +194,14 @@ def loss_mean(loss, n_rows):
     what = "cross_entropy loss_mean"
     dev = _bridge.require_gpu(what, loss)
     n_rows = int(n_rows)
+    if (loss.dtype is torch.float32 and 0 < n_rows <= loss.numel() and loss.is_contiguous() and
+            dev == _raw_device()):
+        out = loss.new_empty_strided((), ())
+        rc = _lib.entry("vbh_reduce_fwd")(loss.data_ptr(), out.data_ptr(), None, 1, n_rows, 1,
+                                          _lib.F32, _lib.F32, _lib.REDUCE_MEAN, _raw_stream(dev))
+        if rc != 0:
+            raise _lib.VbhError("vbh_reduce_fwd", rc, _lib.last_error())
+        return out
     flat = loss.reshape(-1)
     if loss.dtype != torch.float32:
         raise TypeError(f"{what}: loss must be fp32, got {loss.dtype}")

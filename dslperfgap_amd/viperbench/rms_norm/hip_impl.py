@@ -16,11 +16,29 @@ if _ROOT not in sys.path:
 
 import torch  # noqa: E402
 
-from dslperfgap_amd import _bridge  # noqa: E402
+from dslperfgap_amd import _bridge, _lib  # noqa: E402
 
 
 def rms_norm(x, normalized_shape, weight, eps=1e-5):
     """RMS normalization: y = x / sqrt(mean(x^2) + eps) * weight."""
+    # the common call: contiguous x and weight (of x's dtype or fp32) on the
+    # current GPU, normalized over the last dim
+    if type(normalized_shape) is tuple and len(normalized_shape) == 1:
+        key = (x.shape, x.dtype, weight.shape, weight.dtype)
+        p = _PLANS.get(key)
+        if p is None:
+            p = _PLANS.put(key, _plan(*key))
+        if p:
+            dev = x.get_device()
+            if (dev >= 0 and dev == _raw_device() and weight.get_device() == dev and
+                    x.is_contiguous() and weight.is_contiguous()):
+                rows, cols, code, wcode, fn = p
+                y = torch.empty_like(x)
+                rc = fn(x.data_ptr(), weight.data_ptr(), y.data_ptr(), rows, cols, float(eps),
+                        code, wcode, _raw_stream(dev))
+                if rc != 0:
+                    raise _lib.VbhError("vbh_rms_norm_fwd", rc, _lib.last_error())
+                return y
     dev = _bridge.require_gpu("rms_norm", x, weight)
     k = len(tuple(normalized_shape))
     if k > x.dim():
@@ -41,3 +59,19 @@ def rms_norm(x, normalized_shape, weight, eps=1e-5):
     _bridge.launch("vbh_rms_norm_fwd", dev, _bridge.ptr(x), _bridge.ptr(w), _bridge.ptr(y), rows,
                    cols, float(eps), dt, wdt)
     return y
+
+
+# (x shape, dtype, weight shape, dtype) -> (rows, cols, dtype codes, entry point) of
+# a last-dim RMSNorm, or False where a call needs the general path
+_PLANS = _bridge.PlanCache()
+_raw_device, _raw_stream = _bridge._raw_device, _bridge._raw_stream
+
+
+def _plan(shape, dtype, wshape, wdtype):
+    code = _bridge.FLOAT_CODES.get(dtype)
+    if (code is None or len(shape) == 0 or wdtype not in (dtype, torch.float32) or
+            _bridge.numel_prod(wshape) != shape[-1] or shape[-1] == 0):
+        return False
+    cols = int(shape[-1])
+    return (_bridge.numel_prod(shape) // cols, cols, code, _bridge.FLOAT_CODES[wdtype],
+            _lib.entry("vbh_rms_norm_fwd"))
