@@ -634,15 +634,36 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_pipe(
 }
 
 // ---------------------------------------------------------------------------
-// streaming kernels (one 1024-lane workgroup per row, chunked two passes)
+// streaming kernels (one kMaxBlock-lane workgroup per row, two passes)
+//
+// Bound by memory and, with few rows, by one workgroup's loads in flight:
+// kStreamU accesses per lane.  The first pass leaves the row in the caches for
+// the second.  MI355X, one vector in flight -> four: LayerNorm bf16
+// 256 x 131072 44 -> 32 us, fp32 500 x 131072 179 -> 129; RMSNorm bf16
+// 256 x 131072 38 -> 27, fp32 500 x 131072 157 -> 120 (79 at the copy's rate for
+// one read and one write).  Rows read one element per access keep one plain load
+// in flight (four: RMSNorm bf16 600 x 99999 169 -> 182; nontemporal: LayerNorm
+// fp16 20 x 70001 35 -> 42).
 // ---------------------------------------------------------------------------
+constexpr int kStreamU = 4;
+
+// Vectors j0, j0 + kMaxBlock, ... of the row (zero past its end); NT: as load_raw.
+template <typename T, int V, bool NT, int U>
+__device__ __forceinline__ void stream_load(const T* __restrict__ xr, int j0, int nvec,
+                                            typename Raw<T, V>::type (&v)[U], const Span& s) {
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int j = j0 + u * kMaxBlock;
+    if (j < nvec) v[u] = load_raw<T, V, NT>(xr + static_cast<int64_t>(j) * V, s);
+    else v[u] = typename Raw<T, V>::type{};
+  }
+}
 
 template <typename T, typename TW, int V>
 __global__ __launch_bounds__(kMaxBlock) void layer_norm_stream(
     const T* __restrict__ x, const TW* __restrict__ w, const TW* __restrict__ b,
     T* __restrict__ y, int cols, float eps) {
   __shared__ float lds[3 * kMaxWaves];
-  const int tpr = blockDim.x;
   const int nvec = cols / V;
   const int64_t row = blockIdx.x;
   const T* xr = x + row * cols;
@@ -655,37 +676,62 @@ __global__ __launch_bounds__(kMaxBlock) void layer_norm_stream(
   float x0;
   load_f32<T, 1>(xr, &x0, sx);
   Moments m{0.f, 0.f, 0.f};
-  for (int j = threadIdx.x; j < nvec; j += tpr) {
-    float v[V];
-    load_f32<T, V>(xr + static_cast<int64_t>(j) * V, v, sx);
+  constexpr int U = V == 1 ? 1 : kStreamU;
+  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+    typename Raw<T, V>::type v[U];
+    stream_load<T, V, false, U>(xr, j0, nvec, v, sx);
+    // the batch's own two-pass moments, then merged
+    int held = 0;
+    float s[V], q[V];
 #pragma unroll
-    for (int k = 0; k < V; ++k) v[k] -= x0;
-    float s = 0.f;
+    for (int k = 0; k < V; ++k) s[k] = q[k] = 0.f;
 #pragma unroll
-    for (int k = 0; k < V; ++k) s += v[k];
-    const float cm = s / static_cast<float>(V);
-    float q = 0.f;
+    for (int u = 0; u < U; ++u) {
+      if (j0 + u * kMaxBlock < nvec) {
+        ++held;
 #pragma unroll
-    for (int k = 0; k < V; ++k) q = fmaf(v[k] - cm, v[k] - cm, q);
-    m = merge_moments(m, Moments{static_cast<float>(V), cm, q});
+        for (int k = 0; k < V; ++k) s[k] += raw_at<T, V>(v[u], k) - x0;
+      }
+    }
+    const float n = static_cast<float>(held * V);
+    const float cm = tree_sum<V>(s) / n;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (j0 + u * kMaxBlock < nvec) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          const float d = (raw_at<T, V>(v[u], k) - x0) - cm;
+          q[k] = fmaf(d, d, q[k]);
+        }
+      }
+    }
+    m = merge_moments(m, Moments{n, cm, tree_sum<V>(q)});
   }
-  m = group_allreduce_moments(m, tpr, lds);
+  m = group_allreduce_moments(m, kMaxBlock, lds);
   const float mean = m.mean;
   const float rstd = rsqrt_hw(m.m2 * inv_count(cols) + eps);
   T* yr = y + row * cols;
-  for (int j = threadIdx.x; j < nvec; j += tpr) {
-    float v[V], wv[V], bv[V], o[V];
-    load_f32<T, V>(xr + static_cast<int64_t>(j) * V, v, sx);
-    load_f32<TW, V>(w + static_cast<int64_t>(j) * V, wv, sw);
-    if (b != nullptr) {
-      load_f32<TW, V>(b + static_cast<int64_t>(j) * V, bv, sb);
-    } else {
+  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+    typename Raw<T, V>::type v[U];
+    stream_load<T, V, V != 1, U>(xr, j0, nvec, v, sx);
 #pragma unroll
-      for (int k = 0; k < V; ++k) bv[k] = 0.f;
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = j0 + u * kMaxBlock;
+      if (j < nvec) {
+        float wv[V], bv[V], o[V];
+        load_f32<TW, V>(w + j * V, wv, sw);
+        if (b != nullptr) {
+          load_f32<TW, V>(b + j * V, bv, sb);
+        } else {
+#pragma unroll
+          for (int k = 0; k < V; ++k) bv[k] = 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+          o[k] = ((raw_at<T, V>(v[u], k) - x0) - mean) * rstd * wv[k] + bv[k];
+        store_raw<T, V, V != 1>(yr + j * V, o, sy);
+      }
     }
-#pragma unroll
-    for (int k = 0; k < V; ++k) o[k] = ((v[k] - x0) - mean) * rstd * wv[k] + bv[k];
-    store_from_f32<T, V>(yr + static_cast<int64_t>(j) * V, o, sy);
   }
 }
 
@@ -693,8 +739,8 @@ template <typename T, typename TW, int V>
 __global__ __launch_bounds__(kMaxBlock) void rms_norm_stream(
     const T* __restrict__ x, const TW* __restrict__ w, T* __restrict__ y, int cols,
     float eps) {
+  constexpr int U = V == 1 ? 1 : kStreamU;
   __shared__ float lds[kMaxWaves];
-  const int tpr = blockDim.x;
   const int nvec = cols / V;
   const int64_t row = blockIdx.x;
   const T* xr = x + row * cols;
@@ -702,23 +748,37 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_stream(
   const Span sx = VBH_SPAN(x, static_cast<int64_t>(gridDim.x) * cols);
   const Span sy = VBH_SPAN(y, static_cast<int64_t>(gridDim.x) * cols);
   const Span sw = VBH_SPAN(w, cols);
-  float acc = 0.f;
-  for (int j = threadIdx.x; j < nvec; j += tpr) {
-    float v[V];
-    load_f32<T, V>(xr + static_cast<int64_t>(j) * V, v, sx);
+  float acc[V];
 #pragma unroll
-    for (int k = 0; k < V; ++k) acc = fmaf(v[k], v[k], acc);
+  for (int k = 0; k < V; ++k) acc[k] = 0.f;
+  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+    typename Raw<T, V>::type v[U];
+    stream_load<T, V, false, U>(xr, j0, nvec, v, sx);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < V; ++k) {
+        const float f = raw_at<T, V>(v[u], k);
+        acc[k] = fmaf(f, f, acc[k]);
+      }
   }
-  const float ss = group_allreduce<Sum>(acc, tpr, lds);
+  const float ss = group_allreduce<Sum>(tree_sum<V>(acc), kMaxBlock, lds);
   const float rinv = rsqrt_hw(ss * inv_count(cols) + eps);
   T* yr = y + row * cols;
-  for (int j = threadIdx.x; j < nvec; j += tpr) {
-    float v[V], wv[V], o[V];
-    load_f32<T, V>(xr + static_cast<int64_t>(j) * V, v, sx);
-    load_f32<TW, V>(w + static_cast<int64_t>(j) * V, wv, sw);
+  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+    typename Raw<T, V>::type v[U];
+    stream_load<T, V, V != 1, U>(xr, j0, nvec, v, sx);
 #pragma unroll
-    for (int k = 0; k < V; ++k) o[k] = (v[k] * rinv) * wv[k];
-    store_from_f32<T, V>(yr + static_cast<int64_t>(j) * V, o, sy);
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = j0 + u * kMaxBlock;
+      if (j < nvec) {
+        float wv[V], o[V];
+        load_f32<TW, V>(w + j * V, wv, sw);
+#pragma unroll
+        for (int k = 0; k < V; ++k) o[k] = (raw_at<T, V>(v[u], k) * rinv) * wv[k];
+        store_raw<T, V, V != 1>(yr + j * V, o, sy);
+      }
+    }
   }
 }
 
