@@ -327,7 +327,8 @@ __global__ __launch_bounds__(kMaxBlock) void ce_fwd_stream(
 
   // per-thread running max (NaN ignored), rescaled sum, NaN-propagating sum of logits
   float m = kNegInf, s = 0.f, sl = 0.f, nan = 0.f;
-  for (int j = threadIdx.x; j < nvec; j += tpr) {
+  // (unsigned: the last step of a row of almost 2^31 columns passes 2^31)
+  for (uint32_t j = threadIdx.x; j < static_cast<uint32_t>(nvec); j += tpr) {
     float v[V];
     load_f32<T, V>(lr + static_cast<int64_t>(j) * V, v, sx);
     float cm = kNegInf;

@@ -165,16 +165,19 @@ __global__ __launch_bounds__(kMaxBlock) void reduce_rows(const Ti* __restrict__ 
   // processing any of them, so a chunk's loads are in flight together whatever
   // the data-dependent branches below do.
   constexpr int kChunk = 4;
+  // (unsigned vector numbers: in a row of almost 2^31 vectors of one element the
+  // last chunk passes 2^31)
+  const uint32_t nv = nvec;
   if constexpr (OP == 0) {
     float acc[V];
 #pragma unroll
     for (int k = 0; k < V; ++k) acc[k] = 0.f;
-    for (int base = g; base < nvec; base += kChunk * tpr) {
+    for (uint32_t base = g; base < nv; base += kChunk * tpr) {
       RT r[kChunk];
 #pragma unroll
       for (int c = 0; c < kChunk; ++c) {
-        const int j = base + c * tpr;
-        r[c] = j < nvec ? load_raw<Ti, V, true>(xr + static_cast<int64_t>(j) * V, sx) : RT{};
+        const uint32_t j = base + c * tpr;
+        r[c] = j < nv ? load_raw<Ti, V, true>(xr + static_cast<int64_t>(j) * V, sx) : RT{};
       }
 #pragma unroll
       for (int c = 0; c < kChunk; ++c)
@@ -208,21 +211,21 @@ __global__ __launch_bounds__(kMaxBlock) void reduce_rows(const Ti* __restrict__ 
       float bv = kNegInf;  // best vector's maximum
       int bj = -1;         // its vector index (-1: none yet)
       RT braw = RT{};
-      for (int base = g; base < nvec; base += kChunk * tpr) {
+      for (uint32_t base = g; base < nv; base += kChunk * tpr) {
         RT r[kChunk];
 #pragma unroll
         for (int c = 0; c < kChunk; ++c) {
-          const int j = base + c * tpr;
-          r[c] = j < nvec ? load_raw<Ti, V, true>(xr + static_cast<int64_t>(j) * V, sx) : RT{};
+          const uint32_t j = base + c * tpr;
+          r[c] = j < nv ? load_raw<Ti, V, true>(xr + static_cast<int64_t>(j) * V, sx) : RT{};
         }
 #pragma unroll
         for (int c = 0; c < kChunk; ++c) {
-          const int j = base + c * tpr;
-          if (j >= nvec) break;  // the lane's later vectors are past the row too
+          const uint32_t j = base + c * tpr;
+          if (j >= nv) break;  // the lane's later vectors are past the row too
           const float m = vec_max_nan<Ti, V>(r[c]);
           const bool win = bj < 0 || m > bv || (m != m && bv == bv);
           bv = win ? m : bv;
-          bj = win ? j : bj;
+          bj = win ? static_cast<int>(j) : bj;
           braw = win ? r[c] : braw;
         }
       }
@@ -263,17 +266,17 @@ __global__ __launch_bounds__(kMaxBlock) void reduce_rows(const Ti* __restrict__ 
           best = ValIdx{v, g};
         }
       }
-      for (int base = g; base < nvec; base += kChunk * tpr) {
+      for (uint32_t base = g; base < nv; base += kChunk * tpr) {
         RT r[kChunk];
 #pragma unroll
         for (int c = 0; c < kChunk; ++c) {
-          const int j = base + c * tpr;
-          r[c] = j < nvec ? load_raw<Ti, V, true>(xr + static_cast<int64_t>(j) * V, sx) : RT{};
+          const uint32_t j = base + c * tpr;
+          r[c] = j < nv ? load_raw<Ti, V, true>(xr + static_cast<int64_t>(j) * V, sx) : RT{};
         }
 #pragma unroll
         for (int c = 0; c < kChunk; ++c) {
-          const int j = base + c * tpr;
-          if (done || j >= nvec) continue;
+          const uint32_t j = base + c * tpr;
+          if (done || j >= nv) continue;
           float v[V];
 #pragma unroll
           for (int k = 0; k < V; ++k) v[k] = raw_at<Ti, V>(r[c], k);
@@ -289,14 +292,14 @@ __global__ __launch_bounds__(kMaxBlock) void reduce_rows(const Ti* __restrict__ 
 #pragma unroll
             for (int k = V - 1; k >= 0; --k)
               if (v[k] != v[k]) kk = k;
-            best = ValIdx{__builtin_nanf(""), head + j * V + kk};
+            best = ValIdx{__builtin_nanf(""), head + static_cast<int>(j) * V + kk};
             done = true;
           } else if (m > best.v || best.i == n) {  // first position of the vector max
             int kk = V - 1;
 #pragma unroll
             for (int k = V - 1; k >= 0; --k)
               if (v[k] == m) kk = k;
-            best = ValIdx{m, head + j * V + kk};
+            best = ValIdx{m, head + static_cast<int>(j) * V + kk};
           }
         }
       }

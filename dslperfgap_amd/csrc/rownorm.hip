@@ -648,12 +648,14 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_pipe(
 constexpr int kStreamU = 4;
 
 // Vectors j0, j0 + kMaxBlock, ... of the row (zero past its end); NT: as load_raw.
+// Vector numbers are unsigned: in a row of almost 2^31 vectors of one element
+// the last steps pass 2^31.
 template <typename T, int V, bool NT, int U>
-__device__ __forceinline__ void stream_load(const T* __restrict__ xr, int j0, int nvec,
+__device__ __forceinline__ void stream_load(const T* __restrict__ xr, uint32_t j0, uint32_t nvec,
                                             typename Raw<T, V>::type (&v)[U], const Span& s) {
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int j = j0 + u * kMaxBlock;
+    const uint32_t j = j0 + u * kMaxBlock;
     if (j < nvec) v[u] = load_raw<T, V, NT>(xr + static_cast<int64_t>(j) * V, s);
     else v[u] = typename Raw<T, V>::type{};
   }
@@ -664,7 +666,7 @@ __global__ __launch_bounds__(kMaxBlock) void layer_norm_stream(
     const T* __restrict__ x, const TW* __restrict__ w, const TW* __restrict__ b,
     T* __restrict__ y, int cols, float eps) {
   __shared__ float lds[3 * kMaxWaves];
-  const int nvec = cols / V;
+  const uint32_t nvec = static_cast<uint32_t>(cols) / V;
   const int64_t row = blockIdx.x;
   const T* xr = x + row * cols;
   // one workgroup per row: the grid is the row count
@@ -677,7 +679,7 @@ __global__ __launch_bounds__(kMaxBlock) void layer_norm_stream(
   load_f32<T, 1>(xr, &x0, sx);
   Moments m{0.f, 0.f, 0.f};
   constexpr int U = V == 1 ? 1 : kStreamU;
-  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
     typename Raw<T, V>::type v[U];
     stream_load<T, V, false, U>(xr, j0, nvec, v, sx);
     // the batch's own two-pass moments, then merged
@@ -711,7 +713,7 @@ __global__ __launch_bounds__(kMaxBlock) void layer_norm_stream(
   const float mean = m.mean;
   const float rstd = rsqrt_hw(m.m2 * inv_count(cols) + eps);
   T* yr = y + row * cols;
-  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
     typename Raw<T, V>::type v[U];
     stream_load<T, V, V != 1, U>(xr, j0, nvec, v, sx);
 #pragma unroll
@@ -741,7 +743,7 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_stream(
     float eps) {
   constexpr int U = V == 1 ? 1 : kStreamU;
   __shared__ float lds[kMaxWaves];
-  const int nvec = cols / V;
+  const uint32_t nvec = static_cast<uint32_t>(cols) / V;
   const int64_t row = blockIdx.x;
   const T* xr = x + row * cols;
   // one workgroup per row: the grid is the row count
@@ -751,7 +753,7 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_stream(
   float acc[V];
 #pragma unroll
   for (int k = 0; k < V; ++k) acc[k] = 0.f;
-  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
     typename Raw<T, V>::type v[U];
     stream_load<T, V, false, U>(xr, j0, nvec, v, sx);
 #pragma unroll
@@ -765,7 +767,7 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_stream(
   const float ss = group_allreduce<Sum>(tree_sum<V>(acc), kMaxBlock, lds);
   const float rinv = rsqrt_hw(ss * inv_count(cols) + eps);
   T* yr = y + row * cols;
-  for (int j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
     typename Raw<T, V>::type v[U];
     stream_load<T, V, V != 1, U>(xr, j0, nvec, v, sx);
 #pragma unroll

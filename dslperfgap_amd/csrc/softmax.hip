@@ -418,24 +418,25 @@ struct RowStats {
 constexpr int kStreamU = 4;
 
 template <typename T, int V, bool NT>
-__device__ __forceinline__ void stream_load(const T* __restrict__ xr, int j0, int nvec,
+__device__ __forceinline__ void stream_load(const T* __restrict__ xr, uint32_t j0, uint32_t nvec,
                                             typename Raw<T, V>::type (&v)[kStreamU],
                                             const Span& sx) {
   const typename Raw<T, V>::type fill = typename Raw<T, V>::type(static_cast<T>(kNegInf));
 #pragma unroll
   for (int u = 0; u < kStreamU; ++u) {
-    const int j = j0 + u * kMaxBlock;
+    const uint32_t j = j0 + u * kMaxBlock;
     if (j < nvec) v[u] = load_raw<T, V, NT>(xr + static_cast<int64_t>(j) * V, sx);
     else v[u] = fill;
   }
 }
 
-// (the streaming kernels run kMaxBlock lanes per row)
+// (the streaming kernels run kMaxBlock lanes per row; their vector numbers are
+// unsigned: in a row of almost 2^31 vectors of one element the last steps pass 2^31)
 template <typename T, int V, bool NT>
-__device__ __forceinline__ RowStats stream_stats(const T* __restrict__ xr, int nvec,
+__device__ __forceinline__ RowStats stream_stats(const T* __restrict__ xr, uint32_t nvec,
                                                  float* lds, const Span& sx) {
   float m = kNegInf, s = 0.f;
-  for (int j = threadIdx.x; j < nvec; j += kStreamU * kMaxBlock) {
+  for (uint32_t j = threadIdx.x; j < nvec; j += kStreamU * kMaxBlock) {
     typename Raw<T, V>::type v[kStreamU];
     stream_load<T, V, NT>(xr, j, nvec, v, sx);
     const float nm = max_nan(m, lane_max<T, V, kStreamU>(v));
@@ -453,7 +454,7 @@ template <typename Ti, typename To, int V, bool LOG>
 __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const Ti* __restrict__ x,
                                                             To* __restrict__ y, int cols) {
   __shared__ float lds[2 * kMaxWaves];
-  const int nvec = cols / V;
+  const uint32_t nvec = static_cast<uint32_t>(cols) / V;
   const int64_t row = blockIdx.x;
   const Ti* xr = x + row * cols;
   // one workgroup per row: the grid is the row count
@@ -463,12 +464,12 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const Ti* __restrict
   const float m = st.m;
   const float ls = st.special() ? __builtin_nanf("") : (LOG ? fast_log(st.s) : 1.0f / st.s);
   To* yr = y + row * cols;
-  for (int j0 = threadIdx.x; j0 < nvec; j0 += kStreamU * kMaxBlock) {
+  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += kStreamU * kMaxBlock) {
     typename Raw<Ti, V>::type v[kStreamU];
     stream_load<Ti, V, true>(xr, j0, nvec, v, sx);
 #pragma unroll
     for (int u = 0; u < kStreamU; ++u) {
-      const int j = j0 + u * kMaxBlock;
+      const uint32_t j = j0 + u * kMaxBlock;
       if (j < nvec) {
         float o[V];
 #pragma unroll
@@ -487,7 +488,7 @@ template <typename Ti, typename To, int V, bool PAIR = false>
 __global__ __launch_bounds__(kMaxBlock) void logsumexp_stream(const Ti* __restrict__ x,
                                                               To* __restrict__ y, int cols) {
   __shared__ float lds[2 * kMaxWaves];
-  const int nvec = cols / V;
+  const uint32_t nvec = static_cast<uint32_t>(cols) / V;
   const int64_t row = blockIdx.x;
   // one workgroup per row: the grid is the row count
   const Span sx = VBH_SPAN(x, static_cast<int64_t>(gridDim.x) * cols);

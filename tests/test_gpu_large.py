@@ -14,6 +14,7 @@ import torch
 from dslperfgap_amd.viperbench.argmax.hip_impl import argmax
 from dslperfgap_amd.viperbench.cross_entropy.hip_impl import cross_entropy_fwd
 from dslperfgap_amd.viperbench.layer_norm.hip_impl import layer_norm
+from dslperfgap_amd.viperbench.log_softmax.hip_impl import log_softmax
 from dslperfgap_amd.viperbench.logsumexp.hip_impl import logsumexp
 from dslperfgap_amd.viperbench.mean_reduction.hip_impl import mean_reduction
 from dslperfgap_amd.viperbench.rms_norm.hip_impl import rms_norm
@@ -94,3 +95,35 @@ def test_cross_entropy_beyond_2_31_elements():
     idx = torch.tensor(PICK, device=DEV)
     _close(loss.view(-1)[idx], want_loss.view(-1)[:len(PICK)], torch.float32, "loss")
     _close(lse.view(-1)[idx], want_lse.view(-1)[:len(PICK)], torch.float32, "lse")
+
+
+def test_row_of_the_most_columns():
+    """One row of 2^31 - 1 columns (the most an entry point takes, odd, so read
+    one element per access by the streaming kernels): the last steps' vector
+    numbers pass 2^31."""
+    n = 2**31 - 1
+    print(f"[gpu] one row of {n}", flush=True)
+    x = torch.empty(1, n, dtype=torch.float16, device=DEV)
+    x.normal_(generator=torch.Generator(device=DEV).manual_seed(9))
+    x[0, -1] = 9.0  # the last element weighs 8100 of 3.5e9
+    parts = [c.double() for c in (torch.logsumexp(p.float(), 0) for p in x[0].split(1 << 27))]
+    lse = torch.logsumexp(torch.stack(parts), 0).item()
+    # fp32 sums of 2^31 exps, spread over 1024 lanes of 2^21 terms each: the
+    # rounding of a lane's sum is at most 2^21 * 2^-24 of it in the worst case and
+    # its square root in the mean; the fp16 results round to 2^-7 (lse, log_softmax
+    # about 22) and hide both
+    got = logsumexp(x)
+    assert abs(got.item() - lse) < 2**-6
+    print("[gpu] log_softmax", flush=True)
+    y = log_softmax(x, -1)
+    for i in (0, n // 2, n - 5000):
+        want = x[0, i:i + 5000].double() - lse
+        assert (y[0, i:i + 5000].double() - want).abs().max().item() < 2**-6
+    del y
+    print("[gpu] rms_norm", flush=True)
+    w = torch.ones(n, dtype=torch.float16, device=DEV)
+    z = rms_norm(x, (n,), w)
+    ms = sum((p.float() ** 2).sum().double().item() for p in x[0].split(1 << 27)) / n
+    for i in (0, n - 5000):  # fp32 sum of squares as above, then half an fp16 ulp
+        want = x[0, i:i + 5000].double() / (ms + 1e-5) ** 0.5
+        assert torch.allclose(z[0, i:i + 5000].double(), want, atol=1e-3, rtol=4e-3)
