@@ -327,8 +327,7 @@ __global__ __launch_bounds__(kMaxBlock) void ce_fwd_stream(
 
   // per-thread running max (NaN ignored), rescaled sum, NaN-propagating sum of logits
   float m = kNegInf, s = 0.f, sl = 0.f, nan = 0.f;
-  // (unsigned: the last step of a row of almost 2^31 columns passes 2^31)
-  for (uint32_t j = threadIdx.x; j < static_cast<uint32_t>(nvec); j += tpr) {
+  for (int j = threadIdx.x; j < nvec; j += tpr) {
     float v[V];
     load_f32<T, V>(lr + static_cast<int64_t>(j) * V, v, sx);
     float cm = kNegInf;
@@ -442,22 +441,46 @@ struct CeChunk {
 // about 45 us of VALU work against 56 us of memory time for bf16 4096 x 50257
 // -- so they need waves that fold while others wait for loads: one 512-lane
 // workgroup per CU in step takes 129 us there, four of 256 lanes without the
-// barrier 68 (5.9 chunks of 16 KiB in flight per CU; U = 4 or three buffers
-// 72-90).  Vectors at 16-byte boundaries: off them that launch takes 88.
-// MI355X, ce_fwd_rows (ce_fwd_stream at 128256 columns) -> this: bf16
-// 4096 x 50257 93 -> 69 us, with smoothing 132 -> 74; bf16 4096 x 50304 88 -> 69;
-// fp16 4096 x 40000 98 -> 56; bf16 4096 x 128256 191 -> 163; bf16 512 x 50257
-// 15.0 -> 12.9; fp32 4096 x 50257 163 -> 127 (512-lane workgroups, two per CU),
-// with smoothing 175 -> 127.  Rows of up to kCeAnyMinBytes16 / 32 keep ce_fwd_rows,
-// which holds them in half a workgroup's registers: bf16 8192 x 32000 80
-// against 90 us, fp32 8192 x 32001 154 against 161.
+// barrier 68 (chunks of 512 vectors, 8 KiB; U = 4 or three buffers 72-90).
+// Vectors at 16-byte boundaries: off them that launch takes 88.
+// fp32 rows: 512-lane workgroups, two per CU, chunks of 1024 vectors.
+//
+// From kCeAnyMinRows rows of more than kCeAnyMinBytes16 / 32.  MI355X, time of
+// ce_fwd_rows (ce_fwd_stream beyond 65536 16-bit columns) over this, buffers in
+// rotation beyond the caches:
+//   rows                     256   400   512   600  1030  2048  4096  8192
+//   bf16 32776 columns      0.90  1.03  1.07  1.05  1.11  1.10  1.13  1.14
+//   bf16 45056              0.81  0.92  1.00  1.05  1.00  1.04  1.09  1.08
+//   bf16 50257              0.92  1.10  1.18  1.24  1.37  1.36  1.40  1.40
+//   bf16 50257, smoothing   0.99  1.39  1.45  1.60  1.87  1.86  2.01  2.09
+//   bf16 128256             0.95  1.08  1.09  1.31  1.22  1.19  1.18
+//   fp16 45056              0.82  0.88  0.96  0.94  0.97  0.97  1.00  1.04
+//   fp16 50257              0.90  1.06  1.13  1.15  1.29  1.25  1.30  1.30
+//   fp32 50257                          1.27  1.16  1.34  1.34  1.28
+// Rows of up to kCeAnyMinBytes16 / 32 keep ce_fwd_rows, which holds them in
+// half a workgroup's registers: bf16 8192 x 32000 80 against 90 us, fp32
+// 8192 x 32001 154 against 161.
 constexpr int64_t kCeAnyMinRows = 512;
 constexpr int64_t kCeAnyMinBytes16 = int64_t(64) << 10;
 constexpr int64_t kCeAnyMinBytes32 = int64_t(128) << 10;
-// So do aligned 16-bit rows that fill 4 waves of 8 vectors per lane, 8, 12 or
-// 16 of them (bf16 4096 x 65536 84 against 90 us, 1500 x 49152 28.7 against
-// 29.8; but 14 waves, 4096 x 57344, 94 against 79).
-constexpr int64_t kCeAnyFullCols = 16384;
+// ce_fwd_rows also keeps aligned 16-bit rows without smoothing that take 12 or
+// 16 of its waves (8 vectors per lane: kCeWaveCols columns each), as many on
+// each of a CU's four SIMDs: of 16 waves from kCeFullMinRowsBf16 / F16 rows up,
+// and fp16 rows that fill either exactly.  MI355X, as above:
+//   rows                     600  1030  1500  2048  2600  4096  8192
+//   bf16 49152 (12 waves)   1.02  0.99  1.03  0.99  1.02  1.01  1.03
+//   bf16 61440 (15)         1.08  1.01  1.09  1.06  1.08  1.13  1.14
+//   bf16 61448 (16)         1.11  1.02  1.01  0.97  0.99  0.96  0.97
+//   bf16 65536 (16)         1.08  0.98  0.99  0.95  0.96  0.96  0.97
+//   fp16 49144 (12)         0.99  1.05  1.03  1.01  1.01  0.99  0.99
+//   fp16 49152 (12, full)   0.93  0.98  0.97  0.96  0.98  1.00  1.00
+//   fp16 61448 (16)         1.01  0.99  0.97  0.94  0.99  0.96  0.99
+//   fp16 65536 (16, full)   0.99  0.97  0.94  0.90  0.96  0.96  0.96
+// With smoothing (ce_fwd_rows adds up the logits apart) this is the faster one
+// everywhere: 65536 columns bf16 1.12-1.19, fp16 1.06-1.17.
+constexpr int64_t kCeWaveCols = 8 * 8 * kWave;
+constexpr int64_t kCeFullMinRowsBf16 = 2048;
+constexpr int64_t kCeFullMinRowsF16 = 1536;
 
 // SL: the row's sum of scaled logits is needed (smoothing); ONE: logit_scale
 // is 1 (else each logit's product with it is rounded once, as the golden
@@ -1027,12 +1050,17 @@ hipError_t launch_cross_entropy_fwd_persist(const CeArgs& a, int64_t max_grid, i
 
 bool cross_entropy_fwd_any_fits(const CeArgs& a) {
   const bool f32 = a.logits_dt == kF32;
-  if (!f32 && a.n_cols % kCeAnyFullCols == 0 && a.n_cols <= 4 * kCeAnyFullCols &&
-      a.n_rows >= 2 * kCeAnyMinRows && a.ld % 8 == 0 &&
-      (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0)
+  if (a.ncb != 1 || a.n_rows < kCeAnyMinRows || a.n_cols >= (1 << 28) ||
+      a.n_cols * (f32 ? 4 : 2) <= (f32 ? kCeAnyMinBytes32 : kCeAnyMinBytes16))
     return false;
-  return a.ncb == 1 && a.n_rows >= kCeAnyMinRows && a.n_cols < (1 << 28) &&
-         a.n_cols * (f32 ? 4 : 2) > (f32 ? kCeAnyMinBytes32 : kCeAnyMinBytes16);
+  const bool f16 = a.logits_dt == kF16;
+  const int64_t waves = (a.n_cols + kCeWaveCols - 1) / kCeWaveCols;
+  if (f32 || a.has_smoothing || waves % 4 != 0 || waves > kMaxWaves || a.n_cols % 8 != 0 ||
+      a.ld % 8 != 0 || (reinterpret_cast<uintptr_t>(a.logits) & 15u) != 0)
+    return true;
+  const bool full = f16 && a.n_cols % kCeWaveCols == 0;
+  return !full && (waves < kMaxWaves ||
+                   a.n_rows < (f16 ? kCeFullMinRowsF16 : kCeFullMinRowsBf16));
 }
 
 hipError_t launch_cross_entropy_fwd_any(const CeArgs& a, hipStream_t s) {
@@ -1044,14 +1072,19 @@ hipError_t launch_cross_entropy_fwd_any(const CeArgs& a, hipStream_t s) {
     using T = typename decltype(tt)::type;
     constexpr int L = sizeof(T) == 4 ? 512 : 256;
     auto launch = [&](auto kern, auto labels) {
-      const int64_t most = std::max<int64_t>(
-          resident_blocks(reinterpret_cast<const void*>(kern), L, 1024 / L), 1);
-      // as many rows for every workgroup as the busiest one has; 16-bit rows over
-      // up to twice the workgroups where that leaves too few (fp16 1027 x 125120:
-      // 514 of two rows 58 us, 1027 of one 50; fp32 1300 x 50257 42.5 and 47.1)
-      int64_t each = (a.n_rows + most - 1) / most;
-      if (sizeof(T) == 2 && (a.n_rows + each - 1) / each * 8 < most * 7)
-        each = (a.n_rows + 2 * most - 1) / (2 * most);
+      // 16-bit rows: one per workgroup, the next one in as soon as a CU has
+      // room.  Workgroups of equal shares on the resident ones, or on up to
+      // twice as many, wait for the last round: bf16 and fp16, mean of 12
+      // widths, 0.90 of that time at 2100-3100 rows, 0.96 at 4096, 0.92 at
+      // 8192, 1.02 at 2048.  fp32 rows: as many for every workgroup as the
+      // busiest one has (one per workgroup: 0.92 at 600 rows, 1.07 at 800, 0.95
+      // at 1030, 1.04 at 1300, 0.98-1.00 from 2048 up).
+      int64_t each = 1;
+      if constexpr (sizeof(T) == 4) {
+        const int64_t most = std::max<int64_t>(
+            resident_blocks(reinterpret_cast<const void*>(kern), L, 1024 / L), 1);
+        each = (a.n_rows + most - 1) / most;
+      }
       launch_kernel(kern, dim3((a.n_rows + each - 1) / each), dim3(L), 0, s,
                     static_cast<const T*>(a.logits), labels, a.loss, a.lse, a.z_loss, a.n_rows,
                     a.n_cols, a.ld, c);

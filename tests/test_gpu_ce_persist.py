@@ -241,3 +241,32 @@ def test_any_row_cross_entropy_matches_oracle(dtype, rows, cols, pad, offset, pi
           flush=True)
     got = cross_entropy_fwd(xd, labels.to(DEV), **args)
     _check(got, ref.cross_entropy_fwd(logits, labels, **args), rows, f"any {rows}x{cols} {dtype}")
+
+
+# which kernel takes aligned 16-bit rows without smoothing of 12 or 16 of
+# ce_fwd_rows' waves (4096 columns each): True where that kernel keeps them
+KEPT = [(torch.bfloat16, 2048, 65536, True), (torch.bfloat16, 2047, 65536, False),
+        (torch.bfloat16, 2048, 61448, True), (torch.bfloat16, 2048, 61440, False),
+        (torch.bfloat16, 2048, 49152, False), (torch.float16, 1536, 61448, True),
+        (torch.float16, 1535, 61448, False), (torch.float16, 512, 49152, True),
+        (torch.float16, 512, 49144, False), (torch.float16, 512, 65536, True)]
+
+
+@pytest.mark.parametrize("dtype,rows,cols,kept", KEPT)
+@pytest.mark.parametrize("smoothing", [0.0, 0.1])
+def test_which_kernel_takes_full_rows(dtype, rows, cols, kept, smoothing):
+    """The kernels add up a row's exps in other orders, so that lse agrees bit for
+    bit over all rows only where both calls ran the same one."""
+    print(f"[ce persist] kept {rows}x{cols} {dtype} {smoothing}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(970)
+    logits = torch.randn(rows, cols, generator=g, device=DEV).to(dtype)
+    labels = torch.randint(0, cols, (rows,), generator=g, device=DEV)
+    args = (smoothing, 1.0, 0.0, -100, cols, 0, cols, smoothing > 0, False)
+    lse = cross_entropy_fwd(logits, labels, *args)[1].view(-1)[:rows].clone()
+    _lib.tune_override(_lib.OP_CROSS_ENTROPY, 0, 0, _lib.TUNE_NO_PERSIST)
+    try:
+        want = cross_entropy_fwd(logits, labels, *args)[1].view(-1)[:rows].clone()
+    finally:
+        _lib.tune_override(_lib.OP_CROSS_ENTROPY, 0, 0, 0)
+    assert torch.allclose(lse, want, atol=2e-6, rtol=2e-6)
+    assert torch.equal(lse, want) == (kept and smoothing == 0.0)
