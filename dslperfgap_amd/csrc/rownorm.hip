@@ -643,9 +643,22 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_pipe(
 // 256 x 131072 38 -> 27, fp32 500 x 131072 157 -> 120 (79 at the copy's rate for
 // one read and one write).  Rows read one element per access keep one plain load
 // in flight (four: RMSNorm bf16 600 x 99999 169 -> 182; nontemporal: LayerNorm
-// fp16 20 x 70001 35 -> 42).
+// fp16 20 x 70001 35 -> 42).  The second pass loads nontemporally where every
+// row is whole lines (whole_line_rows).
 // ---------------------------------------------------------------------------
 constexpr int kStreamU = 4;
+
+// Whether rows of `cols` elements from x on are whole 128-byte memory lines.  The
+// second pass loads nontemporally only then: of other rows two accesses share the
+// first line of every piece, and a nontemporal one does not keep it for the
+// other.  MI355X, plain -> nontemporal second pass, buffers in rotation beyond
+// the caches / the same ones: RMSNorm bf16 512 x 98304 49 -> 43 us / 43 -> 42.5,
+// but 400 x 100000 43 -> 45 / 36 -> 42.5; LayerNorm fp32 400 x 70000 65 -> 69 /
+// 51 -> 66.  A loop for each policy: one loop with the choice inside lost 2-5%.
+template <typename T>
+__device__ __forceinline__ bool whole_line_rows(const T* x, int cols) {
+  return ((reinterpret_cast<uintptr_t>(x) | static_cast<uint64_t>(cols) * sizeof(T)) & 127) == 0;
+}
 
 // Vectors j0, j0 + kMaxBlock, ... of the row (zero past its end); NT: as load_raw.
 // Vector numbers are unsigned: in a row of almost 2^31 vectors of one element
@@ -713,28 +726,32 @@ __global__ __launch_bounds__(kMaxBlock) void layer_norm_stream(
   const float mean = m.mean;
   const float rstd = rsqrt_hw(m.m2 * inv_count(cols) + eps);
   T* yr = y + row * cols;
-  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
-    typename Raw<T, V>::type v[U];
-    stream_load<T, V, V != 1, U>(xr, j0, nvec, v, sx);
+  auto write_row = [&](auto lines) __attribute__((always_inline)) {
+    for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+      typename Raw<T, V>::type v[U];
+      stream_load<T, V, decltype(lines)::value, U>(xr, j0, nvec, v, sx);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t j = j0 + u * kMaxBlock;
-      if (j < nvec) {
-        float wv[V], bv[V], o[V];
-        load_f32<TW, V>(w + j * V, wv, sw);
-        if (b != nullptr) {
-          load_f32<TW, V>(b + j * V, bv, sb);
-        } else {
+      for (int u = 0; u < U; ++u) {
+        const int64_t j = j0 + u * kMaxBlock;
+        if (j < nvec) {
+          float wv[V], bv[V], o[V];
+          load_f32<TW, V>(w + j * V, wv, sw);
+          if (b != nullptr) {
+            load_f32<TW, V>(b + j * V, bv, sb);
+          } else {
 #pragma unroll
-          for (int k = 0; k < V; ++k) bv[k] = 0.f;
+            for (int k = 0; k < V; ++k) bv[k] = 0.f;
+          }
+#pragma unroll
+          for (int k = 0; k < V; ++k)
+            o[k] = ((raw_at<T, V>(v[u], k) - x0) - mean) * rstd * wv[k] + bv[k];
+          store_raw<T, V, V != 1>(yr + j * V, o, sy);
         }
-#pragma unroll
-        for (int k = 0; k < V; ++k)
-          o[k] = ((raw_at<T, V>(v[u], k) - x0) - mean) * rstd * wv[k] + bv[k];
-        store_raw<T, V, V != 1>(yr + j * V, o, sy);
       }
     }
-  }
+  };
+  if (V != 1 && whole_line_rows(x, cols)) write_row(std::true_type{});
+  else write_row(std::false_type{});
 }
 
 template <typename T, typename TW, int V>
@@ -767,21 +784,25 @@ __global__ __launch_bounds__(kMaxBlock) void rms_norm_stream(
   const float ss = group_allreduce<Sum>(tree_sum<V>(acc), kMaxBlock, lds);
   const float rinv = rsqrt_hw(ss * inv_count(cols) + eps);
   T* yr = y + row * cols;
-  for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
-    typename Raw<T, V>::type v[U];
-    stream_load<T, V, V != 1, U>(xr, j0, nvec, v, sx);
+  auto write_row = [&](auto lines) __attribute__((always_inline)) {
+    for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += U * kMaxBlock) {
+      typename Raw<T, V>::type v[U];
+      stream_load<T, V, decltype(lines)::value, U>(xr, j0, nvec, v, sx);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t j = j0 + u * kMaxBlock;
-      if (j < nvec) {
-        float wv[V], o[V];
-        load_f32<TW, V>(w + j * V, wv, sw);
+      for (int u = 0; u < U; ++u) {
+        const int64_t j = j0 + u * kMaxBlock;
+        if (j < nvec) {
+          float wv[V], o[V];
+          load_f32<TW, V>(w + j * V, wv, sw);
 #pragma unroll
-        for (int k = 0; k < V; ++k) o[k] = (raw_at<T, V>(v[u], k) * rinv) * wv[k];
-        store_raw<T, V, V != 1>(yr + j * V, o, sy);
+          for (int k = 0; k < V; ++k) o[k] = (raw_at<T, V>(v[u], k) * rinv) * wv[k];
+          store_raw<T, V, V != 1>(yr + j * V, o, sy);
+        }
       }
     }
-  }
+  };
+  if (V != 1 && whole_line_rows(x, cols)) write_row(std::true_type{});
+  else write_row(std::false_type{});
 }
 
 // weight dtype: either the activation dtype or fp32
