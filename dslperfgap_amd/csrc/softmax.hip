@@ -415,9 +415,14 @@ struct RowStats {
 // loads there cost bf16 300 x 131072 53 us against 42).  MI355X, one vector in
 // flight -> four: logsumexp fp32 600 x 100000 55 -> 39.5 us, softmax fp32
 // 900 x 131072 268 -> 215, log_softmax fp16 -> fp32 300 x 131072 79 -> 54.
+// The statistics take whole batches without a mask and the last, partial one vector
+// by vector: exps of its filler cost 16-bit rows what the loads in flight had
+// gained (bf16 logsumexp 512 x 81920, 2.5 batches, three buffers in turn: one vector
+// in flight 17.4 us, masked batches 18.8, this 17.3; 2048 x 98304 76 / 65 / 63).
 constexpr int kStreamU = 4;
 
-template <typename T, int V, bool NT>
+// Vectors j0, j0 + kMaxBlock, ... of the row (WHOLE: all in it; else -inf past its end)
+template <typename T, int V, bool NT, bool WHOLE>
 __device__ __forceinline__ void stream_load(const T* __restrict__ xr, uint32_t j0, uint32_t nvec,
                                             typename Raw<T, V>::type (&v)[kStreamU],
                                             const Span& sx) {
@@ -425,7 +430,7 @@ __device__ __forceinline__ void stream_load(const T* __restrict__ xr, uint32_t j
 #pragma unroll
   for (int u = 0; u < kStreamU; ++u) {
     const uint32_t j = j0 + u * kMaxBlock;
-    if (j < nvec) v[u] = load_raw<T, V, NT>(xr + static_cast<int64_t>(j) * V, sx);
+    if (WHOLE || j < nvec) v[u] = load_raw<T, V, NT>(xr + static_cast<int64_t>(j) * V, sx);
     else v[u] = fill;
   }
 }
@@ -436,13 +441,31 @@ template <typename T, int V, bool NT>
 __device__ __forceinline__ RowStats stream_stats(const T* __restrict__ xr, uint32_t nvec,
                                                  float* lds, const Span& sx) {
   float m = kNegInf, s = 0.f;
-  for (uint32_t j = threadIdx.x; j < nvec; j += kStreamU * kMaxBlock) {
-    typename Raw<T, V>::type v[kStreamU];
-    stream_load<T, V, NT>(xr, j, nvec, v, sx);
+  typename Raw<T, V>::type v[kStreamU];
+  auto shift_to = [&]() __attribute__((always_inline)) {  // the max with v, as a shift
     const float nm = max_nan(m, lane_max<T, V, kStreamU>(v));
     const float sh = nm == kNegInf ? 0.f : nm;  // exp(-inf - 0) = 0 instead of NaN
-    s = s * fast_exp(m - sh) + lane_sum_exp<T, V, kStreamU>(v, ExpSub{sh});
+    s *= fast_exp(m - sh);
     m = nm;
+    return ExpSub{sh};
+  };
+  uint32_t j = threadIdx.x;
+  for (uint32_t end = kStreamU * kMaxBlock; end <= nvec; end += kStreamU * kMaxBlock) {
+    stream_load<T, V, NT, true>(xr, j, nvec, v, sx);
+    const ExpSub ex = shift_to();
+    s += lane_sum_exp<T, V, kStreamU>(v, ex);
+    j += kStreamU * kMaxBlock;
+  }
+  if (j < nvec) {  // the last, partial batch: no exps of the filler
+    stream_load<T, V, NT, false>(xr, j, nvec, v, sx);
+    const ExpSub ex = shift_to();
+#pragma unroll
+    for (int u = 0; u < kStreamU; ++u) {
+      if (j + u * kMaxBlock < nvec) {
+        typename Raw<T, V>::type one[1] = {v[u]};
+        s += lane_sum_exp<T, V, 1>(one, ex);
+      }
+    }
   }
   const float gm = group_allreduce<Max>(m, kMaxBlock, lds);
   const float t = m == kNegInf ? 0.f : s * fast_exp(m - gm);
@@ -466,7 +489,7 @@ __global__ __launch_bounds__(kMaxBlock) void softmax_stream(const Ti* __restrict
   To* yr = y + row * cols;
   for (uint32_t j0 = threadIdx.x; j0 < nvec; j0 += kStreamU * kMaxBlock) {
     typename Raw<Ti, V>::type v[kStreamU];
-    stream_load<Ti, V, true>(xr, j0, nvec, v, sx);
+    stream_load<Ti, V, true, false>(xr, j0, nvec, v, sx);
 #pragma unroll
     for (int u = 0; u < kStreamU; ++u) {
       const uint32_t j = j0 + u * kMaxBlock;
