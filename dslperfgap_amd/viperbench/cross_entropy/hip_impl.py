@@ -51,8 +51,9 @@ def _logits(logits, what):
 
 _raw_device, _raw_stream = _bridge._raw_device, _bridge._raw_stream
 # (logits shape, dtype, labels shape, dtype, BLOCK_SIZE) -> (rows, columns, logits
-# code, label code, entry point), or False where a call needs the general path
-# (which raises the errors of invalid calls)
+# code, label code, entry point, and of the forward workspace bytes (0: rows not
+# split)), or False where a call needs the general path (which raises the errors of
+# invalid calls)
 _FWD_PLANS = _bridge.PlanCache()
 _BWD_PLANS = _bridge.PlanCache()
 
@@ -67,9 +68,10 @@ def _shape_plan(shape, dtype, lshape, ldtype, block):
 
 def _fwd_plan(shape, dtype, lshape, ldtype, block):
     p = _shape_plan(shape, dtype, lshape, ldtype, block)
-    if not p or _lib.cross_entropy_workspace_bytes(p[0], p[1], block, p[2]):
+    if not p:
         return False
-    return (*p, _lib.entry("vbh_cross_entropy_fwd"))
+    ws_bytes = _lib.cross_entropy_workspace_bytes(p[0], p[1], block, p[2])
+    return (*p, _lib.entry("vbh_cross_entropy_fwd_ws"), ws_bytes)
 
 
 def _bwd_plan(shape, dtype, lshape, ldtype, block):
@@ -82,8 +84,8 @@ def cross_entropy_fwd(
     ignored_index, total_classes, class_start_idx, BLOCK_SIZE, HAS_SMOOTHING, SPLIT
 ):
     """Column-blocked CE forward; see the module docstring for the layout."""
-    # the common call: contiguous logits and labels on the current GPU, rows not
-    # split -- one pass over the tensors' attributes, a cached plan per shape
+    # the common call: contiguous logits and labels on the current GPU -- one pass
+    # over the tensors' attributes, a cached plan per shape
     if type(BLOCK_SIZE) is int:
         key = (logits.shape, logits.dtype, labels.shape, labels.dtype, BLOCK_SIZE)
         p = _FWD_PLANS.get(key)
@@ -93,17 +95,20 @@ def cross_entropy_fwd(
             dev = logits.get_device()
             if (dev >= 0 and dev == _raw_device() and labels.get_device() == dev and
                     logits.is_contiguous() and labels.is_contiguous()):
-                n_rows, n_cols, code, lcode, fn = p
+                n_rows, n_cols, code, lcode, fn, ws_bytes = p
                 loss = torch.empty_like(logits, dtype=torch.float32)
                 lse = torch.empty_like(loss)
                 z_loss = torch.empty_like(loss)
+                # few long rows in one column block: split each row over workgroups
+                ws = _bridge.empty(logits, (ws_bytes,), torch.uint8) if ws_bytes else None
                 rc = fn(logits.data_ptr(), labels.data_ptr(), code, lcode, loss.data_ptr(),
                         lse.data_ptr(), z_loss.data_ptr(), n_rows, n_cols, n_cols,
                         float(smoothing), float(logit_scale), float(lse_square_scale),
                         int(ignored_index), int(total_classes), int(class_start_idx), BLOCK_SIZE,
-                        int(bool(HAS_SMOOTHING)), int(bool(SPLIT)), _raw_stream(dev))
+                        int(bool(HAS_SMOOTHING)), int(bool(SPLIT)),
+                        ws.data_ptr() if ws_bytes else None, ws_bytes, _raw_stream(dev))
                 if rc != 0:
-                    raise _lib.VbhError("vbh_cross_entropy_fwd", rc, _lib.last_error())
+                    raise _lib.VbhError("vbh_cross_entropy_fwd_ws", rc, _lib.last_error())
                 return loss, lse, z_loss
     what = "cross_entropy_fwd"
     dev = _bridge.require_gpu(what, logits, labels)

@@ -125,3 +125,20 @@ def test_reductions_reject_an_empty_reduced_axis():
             fn()
     with pytest.raises(IndexError, match="Dimension out of range"):
         mx.max_reduction(torch.empty(2, 3), 2)
+
+
+def test_split_calls_have_a_plan():
+    """Calls whose rows the library splits (a workspace) are planned like the others."""
+    from dslperfgap_amd import _lib
+
+    lse = _load("logsumexp")
+    for shape, split in (((8, 131072), True), ((131072,), True), ((8, 1024), False)):
+        p = lse._plan(torch.empty(shape), torch.float32)
+        rows = shape[0] if len(shape) == 2 else 1
+        assert (p[4] > 0) == split
+        assert p[4] == _lib.logsumexp_workspace_bytes(rows, shape[-1], _lib.F32)
+    ce = _load("cross_entropy")
+    for cols, block, split in ((131072, 131072, True), (131072, 1024, False), (1024, 1024, False)):
+        p = ce._fwd_plan((8, cols), torch.float32, (8,), torch.int64, block)
+        assert (p[5] > 0) == split
+        assert p[5] == _lib.cross_entropy_workspace_bytes(8, cols, block, _lib.F32)
