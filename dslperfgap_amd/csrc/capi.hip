@@ -593,8 +593,31 @@ ColGeometry softmax_col_geometry(int64_t outer, int64_t n, int64_t inner, int es
   if (c.block == kColBlock) {
     const int wave_lines = std::max(kWave / c.cx, 1);
     c.rows = lines_for(4) <= wave_lines ? 4 : lines_for(8) <= wave_lines ? 8 : 16;
+// Axes of up to 10 (16-bit outputs: 16) run one lane per column
+// (softmax_short_cols) in launches that move up to kSmShortBytes, and beyond that
+// in narrow slabs.  MI355X, log_softmax, device time per call, tiles -> one lane
+// per column: fp16 64 x 2 x 512 4.5 -> 2.6 us, bf16 -> fp32 87381 x 4 x 6
+// 13.1 -> 6.1, fp16 2097152 x 2 x 2 104 -> 12.9, 65536 x 4 x 32 15.8 -> 10.5,
+// 104857 x 10 x 8 24.6 -> 13.2; but fp16 131072 x 4 x 64 31.7 -> 53.3 and fp32
+// 349525 x 8 x 12 49.3 -> 63.5.
+constexpr int64_t kSmShortBytes = int64_t(24) << 20;
+
+bool softmax_short_axis(int64_t outer, int64_t n, int64_t inner, int esize, int osize) {
+  const int size = std::max(esize, osize), vn = 16 / size;
+  if (inner < vn) return n <= (vn == 8 ? 8 : 6);
+  if (n > (vn == 8 ? 16 : 10)) return false;
+  if (mul_sat(mul_sat(outer, inner), n * (esize + osize)) <= kSmShortBytes) return true;
+  return n <= 10 && inner * size <= 96 && n * inner * size <= 256;
+}
+
     if (c.rows > 4 && fits(4, kColBlock) &&
         mul_sat(units(), int64_t(lines_for(c.rows)) * c.cx) < 512 * kColBlock)
+  if (softmax_short_axis(outer, n, inner, esize, osize)) {
+    c.short_axis = true;
+    c.rows = n <= 4 ? 4 : n <= 8 ? 8 : 16;
+    c.grid = (mul_sat(outer, inner) + kColBlock - 1) / kColBlock;
+    return c;
+  }
       c.rows = 4;
   } else {
     c.rows = fits(8, kMaxBlock) ? 8 : fits(16, kMaxBlock) ? 16 : 0;
