@@ -59,13 +59,6 @@ std::atomic<int> g_tpr[kNumOps];
 std::atomic<int> g_block[kNumOps];
 std::atomic<int> g_flags[kNumOps];
 
-// a * b for sizes (a, b >= 0), saturated at INT64_MAX: products of caller
-// sizes are formed before the range checks that reject them.
-int64_t mul_sat(int64_t a, int64_t b) {
-  int64_t r;
-  return __builtin_mul_overflow(a, b, &r) ? INT64_MAX : r;
-}
-
 // Built-in choices per op, from launch-shape sweeps on MI355X:
 //   vectors per lane before more lanes are added (pick_geometry): 2 for RMSNorm
 //   and fp32 softmax, 4 for 16-bit softmax (bf16 8192 columns: +8% over 2),
@@ -106,18 +99,7 @@ constexpr int64_t kShortRowVecs = 32;
 constexpr int kItShort[kNumOps] = {2, 2, 2, 2, 4, 4};
 constexpr int kMinLanesShort[kNumOps] = {4, 8, 8, 8, 2, 4};
 
-// 16-bit softmax rows written as fp32 (8-byte vectors): launches of this many
-// elements or more choose by row width more finely (it_target, mixed_eight)
-constexpr int64_t kMixedManyElems = int64_t(1) << 21;
-
-int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in, int64_t units) {
-  // 16-bit softmax rows written as fp32, 9-12 vectors: 8 lanes of 2, and 16 lanes
-  // of 1 only in small launches.  MI355X, 16 -> 8 lanes, fp16 / bf16 at 2^25
-  // elements: 36 columns 59.0 -> 42.3 / 61.4 -> 42.3 us, 44 columns 52.2 -> 44.4 /
-  // 52.9 -> 45.3; at 2^20 3.68 -> 3.87 / 3.79 -> 3.98.
-  if (op == VBH_OP_SOFTMAX && half_in && vec == 4 && nvec > 8 && nvec <= 12 &&
-      mul_sat(units, nvec * vec) >= kMixedManyElems)
-    return 2;
+int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in) {
   if (vec > 1 && nvec <= kShortRowVecs) {
     int it = kItShort[op];
     while (it > 1 && nvec / it < kMinLanesShort[op]) it /= 2;
@@ -129,14 +111,6 @@ int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in, i
   // the 8-byte vectors of 16-bit rows written as fp32 (bf16 20000 x 255 at 1 / 2
   // / 4 vectors 9.6 / 9.0 / 7.3 us, fp16 50000 x 135 17.2 / 12.8 / 12.7)
   if (op == VBH_OP_SOFTMAX && vec == 4 && nvec <= kWave) return half_in ? 4 : 1;
-  // and 4 of them from 129 vectors up, but 2 in rows of up to 512 that fill every
-  // wave at 2 (fp16 2^23 / 2^25 elements, us at 2 -> 4 per lane: 569 columns
-  // 15.4 -> 11.4 / 53.9 -> 36.8, 2560 11.1 -> 10.6 / 37.7 -> 33.8, 4096
-  // 10.4 -> 8.5 / 34.6 -> 34.4, 8192 11.0 -> 8.3 / 40.4 -> 34.6; but 448 columns
-  // 10.2 -> 10.8 / 32.3 -> 34.1 and 1024 9.9 -> 8.5 / 32.8 -> 34.6)
-  if (op == VBH_OP_SOFTMAX && vec == 4 && half_in && nvec > 2 * kWave &&
-      !(nvec <= 8 * kWave && nvec % (2 * kWave) == 0))
-    return 4;
   // 16-bit LayerNorm rows of 1025-1536 vectors: 2 vectors per lane, 9-12 waves
   // per row (bf16 at 64 MB per call, 4 -> 2: 9216 columns 4298 -> 5247 GB/s,
   // 10240 4501 -> 5194, 11264 4855 -> 5199, 12288 5126 -> 5290; at 768 and
@@ -191,6 +165,13 @@ int pow2ceil(int64_t n) {
   int p = 1;
   while (p < n) p <<= 1;
   return p;
+}
+
+// a * b for sizes (a, b >= 0), saturated at INT64_MAX: products of caller
+// sizes are formed before the range checks that reject them.
+int64_t mul_sat(int64_t a, int64_t b) {
+  int64_t r;
+  return __builtin_mul_overflow(a, b, &r) ? INT64_MAX : r;
 }
 
 int row_group_lanes(int64_t nvec, int it) {
@@ -350,8 +331,7 @@ Geometry geometry_for(int op, int64_t cols, int vec, int64_t units, int64_t out_
   const int64_t nvec = cols / vec;
   const bool half_in = dtype == kF16 || dtype == kBF16;
   Geometry g =
-      pick_geometry(cols, vec,
-                    fill_it(it_target(op, nvec, vec, column_blocks, half_in, units), nvec, units),
+      pick_geometry(cols, vec, fill_it(it_target(op, nvec, vec, column_blocks, half_in), nvec, units),
                     g_tpr[op].load(), g_block[op].load(), flags);
   if (g.persist && !(over & kFlagPersist) && g.tpr < kPersistMinTpr[op]) g.persist = false;
   // LayerNorm row groups of exactly 2 waves run 4 to a 512-lane workgroup
@@ -441,8 +421,7 @@ Geometry reduce_geometry(int64_t n, int vec, int64_t units) {
   const int64_t nvec = n / vec;
   int tpr = g_tpr[VBH_OP_REDUCE].load();
   if (tpr <= 0) {
-    const int per_lane =
-        fill_it(it_target(VBH_OP_REDUCE, nvec, vec, false, false, units), nvec, units);
+    const int per_lane = fill_it(it_target(VBH_OP_REDUCE, nvec, vec, false, false), nvec, units);
     const int64_t lanes = (nvec + per_lane - 1) / per_lane;
     if (lanes <= kWave) {
       tpr = pow2ceil(lanes < 1 ? 1 : lanes);
@@ -494,7 +473,7 @@ constexpr int64_t kColSplitRows = 64;
 constexpr int kColSplitLines = 16;
 
 ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int esize,
-                         int op, bool can_split) {
+                         bool can_split) {
   ColGeometry c;
   c.v = inner >= vn ? vn : 1;
   const int64_t cv = (inner + c.v - 1) / c.v;
@@ -514,52 +493,9 @@ ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int es
   c.segs = 1;
   if (can_split && n / lines >= kColSplitRows &&
       grid_at(lines) < (cv < 8 ? kColSplitGridNarrow : large ? kColGridLarge : kColSplitGrid)) {
-// Short axes run one lane per column (reduce_short_cols): a tile of few rows
-// pays for its exchange through LDS, and leaves a small launch few workgroups.
-// MI355X, device time per call, tiles -> one lane per column:
-//   up to kShortAxisElems elements: mean bf16 1310 x 4 x 100 4.4 -> 2.7 us,
-//   10922 x 12 x 16 4.1 -> 3.3, mean fp32 32768 x 8 x 8 3.7 -> 3.1, means of up to
-//   a quarter of that 3276 x 10 x 16 3.3 -> 2.9, max fp32 of 4 or fewer up to four
-//   times 131072 x 4 x 16 14.4 -> 12.8; but mean bf16 8192 x 8 x 128 6.0 -> 8.1;
-//   narrow slabs (rows under 16 bytes): max bf16 74898 x 16 x 7 16.1 -> 10.2 us,
-//   233016 x 24 x 6 44.7 -> 36.2, mean bf16 2097152 x 4 x 4 43.5 -> 23.0, fp32
-//   3728270 x 3 x 3 57.0 -> 44.9; but max bf16 349525 x 24 x 4 39.2 -> 42.1,
-//   1048576 x 16 x 2 46.8 -> 66.2, mean fp32 1864135 x 6 x 3 35.4 -> 45.3.
-constexpr int64_t kShortAxisElems = int64_t(1) << 21;
-
-bool reduce_short_axis(int64_t outer, int64_t n, int64_t inner, int vn, int op) {
-  const bool half = vn == 8;
-  const int64_t elems = mul_sat(mul_sat(outer, inner), n);
-  if (inner >= vn) {
-    if (!half && op != 0 && n <= 4 && inner >= 16) return elems <= 4 * kShortAxisElems;
-    const bool long_axis = half || (op == 0 && elems <= kShortAxisElems / 4);
-    return n <= (long_axis ? 12 : 8) && elems <= kShortAxisElems;
-  }
-  if (n <= (half ? 10 : 4)) return true;
-  if (!half) return n <= 6 && elems <= kShortAxisElems;
-  return inner > 2 && elems >= kShortAxisElems / 2 &&
-         n <= (inner > 4 && elems >= 3 * kShortAxisElems ? 24 : 16);
-}
-
-// Tiles load nontemporally where a row of the slab is at least this long (half of
-// it over longer axes).  In narrower slabs several accesses share each line, and
-// a nontemporal one does not keep it for the others.  MI355X, nontemporal -> plain:
-// mean bf16 699050 x 6 x 8 39.5 -> 18.3 us, 233016 x 48 x 3 37.8 -> 21.9, max bf16
-// 524288 x 4 x 16 41.1 -> 32.4, mean fp32 1198372 x 4 x 7 55.4 -> 35.0; but mean fp32
-// 87381 x 24 x 16 22.9 -> 25.9, 174762 x 24 x 8 22.6 -> 25.8, max bf16
-// 5461 x 24 x 64 6.9 -> 7.4.
-constexpr int64_t kColNtBytes = 64;
-constexpr int64_t kColNtLongAxis = 24;
-
     lines = c.cx >= 8 ? std::min(most, kColSplitLines) : most;
     while (c.segs < kColMaxSegs && grid_at(lines) * c.segs < kColSplitTarget &&
            n / (int64_t(c.segs) * 2 * lines) >= 8)
-  if (reduce_short_axis(outer, n, inner, vn, op)) {
-    c.short_axis = true;
-    c.grid = (mul_sat(outer, inner) + kColBlock - 1) / kColBlock;
-    return c;
-  }
-  c.nt = inner * esize >= (n < kColNtLongAxis ? kColNtBytes : kColNtBytes / 2);
       c.segs *= 2;
   }
   if (grid_at(lines) > kMaxWorkItems / kColBlock) {  // billions of columns: one lane each
@@ -614,31 +550,8 @@ ColGeometry softmax_col_geometry(int64_t outer, int64_t n, int64_t inner, int es
   if (c.block == kColBlock) {
     const int wave_lines = std::max(kWave / c.cx, 1);
     c.rows = lines_for(4) <= wave_lines ? 4 : lines_for(8) <= wave_lines ? 8 : 16;
-// Axes of up to 10 (16-bit outputs: 16) run one lane per column
-// (softmax_short_cols) in launches that move up to kSmShortBytes, and beyond that
-// in narrow slabs.  MI355X, log_softmax, device time per call, tiles -> one lane
-// per column: fp16 64 x 2 x 512 4.5 -> 2.6 us, bf16 -> fp32 87381 x 4 x 6
-// 13.1 -> 6.1, fp16 2097152 x 2 x 2 104 -> 12.9, 65536 x 4 x 32 15.8 -> 10.5,
-// 104857 x 10 x 8 24.6 -> 13.2; but fp16 131072 x 4 x 64 31.7 -> 53.3 and fp32
-// 349525 x 8 x 12 49.3 -> 63.5.
-constexpr int64_t kSmShortBytes = int64_t(24) << 20;
-
-bool softmax_short_axis(int64_t outer, int64_t n, int64_t inner, int esize, int osize) {
-  const int size = std::max(esize, osize), vn = 16 / size;
-  if (inner < vn) return n <= (vn == 8 ? 8 : 6);
-  if (n > (vn == 8 ? 16 : 10)) return false;
-  if (mul_sat(mul_sat(outer, inner), n * (esize + osize)) <= kSmShortBytes) return true;
-  return n <= 10 && inner * size <= 96 && n * inner * size <= 256;
-}
-
     if (c.rows > 4 && fits(4, kColBlock) &&
         mul_sat(units(), int64_t(lines_for(c.rows)) * c.cx) < 512 * kColBlock)
-  if (softmax_short_axis(outer, n, inner, esize, osize)) {
-    c.short_axis = true;
-    c.rows = n <= 4 ? 4 : n <= 8 ? 8 : 16;
-    c.grid = (mul_sat(outer, inner) + kColBlock - 1) / kColBlock;
-    return c;
-  }
       c.rows = 4;
   } else {
     c.rows = fits(8, kMaxBlock) ? 8 : fits(16, kMaxBlock) ? 16 : 0;
@@ -992,26 +905,6 @@ RowSplit softmax_split(int64_t rows, int64_t cols, int vn) {
   return RowSplit{static_cast<int>((cols + seg_cols - 1) / seg_cols), seg_cols};
 }
 
-namespace {
-
-// Whether 16-bit rows written as fp32 take 8 elements per lane access after all:
-// short rows that then have one access per lane and half the lanes, in launches
-// of kMixedManyElems or more.  MI355X, 4 -> 8 elements, fp16 / bf16 at 2^25
-// elements: 24 columns 48.3 -> 38.4 / 50.6 -> 39.1 us, 40 54.3 -> 38.8 /
-// 57.3 -> 39.7, 56 43.6 -> 37.7 / 45.1 -> 38.8, 41 69.0 -> 54.6 / 74.1 -> 58.0,
-// 65 60.8 -> 51.9 / 58.6 -> 52.0 (at 2^23 14.4 -> 15.7), at 2^22 40 9.0 -> 7.6 /
-// 9.0 -> 7.5; but 64 34.5 -> 38.5 / 34.0 -> 38.9, 35 50.1 -> 56.7 /
-// 52.5 -> 61.3, 52 45.5 -> 48.2 / 47.3 -> 48.5 and, at 2^20, 24 columns 3.53 -> 3.77.
-bool mixed_eight(int64_t rows, int64_t cols) {
-  const int64_t elems = mul_sat(rows, cols);
-  if (g_tpr[VBH_OP_SOFTMAX].load() || g_block[VBH_OP_SOFTMAX].load() || elems < kMixedManyElems)
-    return false;
-  if (cols % 8 == 0) return cols >= 24 && cols < 64;
-  return cols % 4 != 0 && cols > 36 && cols < (elems < 8 * kMixedManyElems ? 64 : 68);
-}
-
-}  // namespace
-
 int64_t vbh_softmax_workspace_bytes(int64_t rows, int64_t cols, int in_dtype) {
   if (!is_float(in_dtype) || rows <= 0 || cols <= 0 || cols > kMaxCols) return 0;
   const int vn = 16 / elt_size(in_dtype);
@@ -1036,8 +929,7 @@ int vbh_softmax_fwd_ws(const void* x, void* y, int64_t rows, int64_t cols, int i
   if (rows == 0 || cols == 0) return 0;
   if (!x || !y) return fail(VBH_E_INVALID, "softmax: null pointer");
   const int vn = 16 / elt_size(in_dtype);
-  // elements per lane access of the kernels that write y
-  const int vo = mixed_eight(rows, cols) ? vn : std::min(vn, 16 / elt_size(out_dtype));
+  const int vo = std::min(vn, 16 / elt_size(out_dtype));  // of the kernels that write y
   const bool aligned = aligned16(x) && aligned16(y);
   const bool vec_ok = cols % vo == 0 && aligned;
   const bool mis_ok = !vec_ok && aligned && cols >= kMisMinVecs * vo;
@@ -1414,7 +1306,7 @@ int64_t vbh_reduce_workspace_bytes(int64_t outer, int64_t n, int64_t inner, int 
   const int vn = 16 / elt_size(in_dtype);
   if (inner > 1) {
     if (mul_sat(outer, inner) > kMaxWorkItems / 256 * 256) return 0;
-    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), op, true);
+    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), true);
     return c.segs > 1 ? outer * inner * c.segs * (op == 0 ? 4 : 8) : 0;
   }
   if (n % vn != 0 || g_tpr[VBH_OP_REDUCE].load() || g_block[VBH_OP_REDUCE].load()) return 0;
@@ -1482,11 +1374,10 @@ int vbh_reduce_fwd_ws(const void* x, void* values, void* indices, int64_t outer,
     const int64_t need = vbh_reduce_workspace_bytes(outer, n, inner, in_dtype, op);
     const bool split = need > 0 && workspace != nullptr && workspace_bytes >= need &&
                        aligned16(workspace);
-    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), op, split);
-    return hip_status(
-        launch_reduce_cols(x, values, idx, split ? workspace : nullptr, outer,
-                           static_cast<int>(n), inner, in_dtype, out_dtype, op, c, s),
-        "reduce launch");
+    return hip_status(launch_reduce_cols(x, values, idx, split ? workspace : nullptr, outer,
+                                         static_cast<int>(n), inner, in_dtype, out_dtype, op,
+                                         col_geometry(outer, n, inner, vn, elt_size(in_dtype), split), s),
+                      "reduce launch");
   }
   return hip_status(launch_reduce(x, values, idx, outer, static_cast<int>(n), in_dtype,
                                   out_dtype, op, g, s),
