@@ -472,9 +472,52 @@ constexpr int64_t kColSplitTarget = 256;
 constexpr int64_t kColSplitRows = 64;
 constexpr int kColSplitLines = 16;
 
+// Short axes run one lane per column (reduce_short_cols): a tile of few rows
+// pays for its exchange through LDS, and leaves a small launch few workgroups.
+// MI355X, device time per call, tiles -> one lane per column:
+//   up to kShortAxisElems elements: mean bf16 1310 x 4 x 100 4.4 -> 2.7 us,
+//   10922 x 12 x 16 4.1 -> 3.3, mean fp32 32768 x 8 x 8 3.7 -> 3.1, means of up to
+//   a quarter of that 3276 x 10 x 16 3.3 -> 2.9, max fp32 of 4 or fewer up to four
+//   times 131072 x 4 x 16 14.4 -> 12.8; but mean bf16 8192 x 8 x 128 6.0 -> 8.1;
+//   narrow slabs (rows under 16 bytes): max bf16 74898 x 16 x 7 16.1 -> 10.2 us,
+//   233016 x 24 x 6 44.7 -> 36.2, mean bf16 2097152 x 4 x 4 43.5 -> 23.0, fp32
+//   3728270 x 3 x 3 57.0 -> 44.9; but max bf16 349525 x 24 x 4 39.2 -> 42.1,
+//   1048576 x 16 x 2 46.8 -> 66.2, mean fp32 1864135 x 6 x 3 35.4 -> 45.3.
+constexpr int64_t kShortAxisElems = int64_t(1) << 21;
+
+bool reduce_short_axis(int64_t outer, int64_t n, int64_t inner, int vn, int op) {
+  const bool half = vn == 8;
+  const int64_t elems = mul_sat(mul_sat(outer, inner), n);
+  if (inner >= vn) {
+    if (!half && op != 0 && n <= 4 && inner >= 16) return elems <= 4 * kShortAxisElems;
+    const bool long_axis = half || (op == 0 && elems <= kShortAxisElems / 4);
+    return n <= (long_axis ? 12 : 8) && elems <= kShortAxisElems;
+  }
+  if (n <= (half ? 10 : 4)) return true;
+  if (!half) return n <= 6 && elems <= kShortAxisElems;
+  return inner > 2 && elems >= kShortAxisElems / 2 &&
+         n <= (inner > 4 && elems >= 3 * kShortAxisElems ? 24 : 16);
+}
+
+// Tiles load nontemporally where a row of the slab is at least this long (half of
+// it over longer axes).  In narrower slabs several accesses share each line, and
+// a nontemporal one does not keep it for the others.  MI355X, nontemporal -> plain:
+// mean bf16 699050 x 6 x 8 39.5 -> 18.3 us, 233016 x 48 x 3 37.8 -> 21.9, max bf16
+// 524288 x 4 x 16 41.1 -> 32.4, mean fp32 1198372 x 4 x 7 55.4 -> 35.0; but mean fp32
+// 87381 x 24 x 16 22.9 -> 25.9, 174762 x 24 x 8 22.6 -> 25.8, max bf16
+// 5461 x 24 x 64 6.9 -> 7.4.
+constexpr int64_t kColNtBytes = 64;
+constexpr int64_t kColNtLongAxis = 24;
+
 ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int esize,
-                         bool can_split) {
+                         int op, bool can_split) {
   ColGeometry c;
+  if (reduce_short_axis(outer, n, inner, vn, op)) {
+    c.short_axis = true;
+    c.grid = (mul_sat(outer, inner) + kColBlock - 1) / kColBlock;
+    return c;
+  }
+  c.nt = inner * esize >= (n < kColNtLongAxis ? kColNtBytes : kColNtBytes / 2);
   c.v = inner >= vn ? vn : 1;
   const int64_t cv = (inner + c.v - 1) / c.v;
   const int64_t bytes = mul_sat(mul_sat(outer, n), mul_sat(inner, esize));
@@ -1306,7 +1349,7 @@ int64_t vbh_reduce_workspace_bytes(int64_t outer, int64_t n, int64_t inner, int 
   const int vn = 16 / elt_size(in_dtype);
   if (inner > 1) {
     if (mul_sat(outer, inner) > kMaxWorkItems / 256 * 256) return 0;
-    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), true);
+    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), op, true);
     return c.segs > 1 ? outer * inner * c.segs * (op == 0 ? 4 : 8) : 0;
   }
   if (n % vn != 0 || g_tpr[VBH_OP_REDUCE].load() || g_block[VBH_OP_REDUCE].load()) return 0;
@@ -1374,10 +1417,11 @@ int vbh_reduce_fwd_ws(const void* x, void* values, void* indices, int64_t outer,
     const int64_t need = vbh_reduce_workspace_bytes(outer, n, inner, in_dtype, op);
     const bool split = need > 0 && workspace != nullptr && workspace_bytes >= need &&
                        aligned16(workspace);
-    return hip_status(launch_reduce_cols(x, values, idx, split ? workspace : nullptr, outer,
-                                         static_cast<int>(n), inner, in_dtype, out_dtype, op,
-                                         col_geometry(outer, n, inner, vn, elt_size(in_dtype), split), s),
-                      "reduce launch");
+    const ColGeometry c = col_geometry(outer, n, inner, vn, elt_size(in_dtype), op, split);
+    return hip_status(
+        launch_reduce_cols(x, values, idx, split ? workspace : nullptr, outer,
+                           static_cast<int>(n), inner, in_dtype, out_dtype, op, c, s),
+        "reduce launch");
   }
   return hip_status(launch_reduce(x, values, idx, outer, static_cast<int>(n), in_dtype,
                                   out_dtype, op, g, s),

@@ -6,7 +6,8 @@
 //   registers and any n works), then all-reduce across the group.
 //   inner > 1: column tiles (col_lane): each lane owns the columns of one
 //   16-byte vector and takes every 2^ty_log2-th row, the lines of lanes are
-//   combined through LDS; few columns split the axis over workgroups.
+//   combined through LDS; few columns split the axis over workgroups; short
+//   axes of small launches or narrow slabs run one lane per column.
 // Each input element is read once; one value (and/or index) per output is
 // written.
 //
@@ -361,7 +362,7 @@ __global__ __launch_bounds__(256) void reduce_combine_vi(const T* __restrict__ p
 // through LDS to the lanes that write them, so that stores of consecutive
 // columns coalesce (straight from the lanes, the int64 indices of one lane are
 // 64 bytes apart: max fp32 3375 x 3 x 512 12.9 against 8.7 us).
-template <typename Ti, typename To, int V, int OP, bool PART>
+template <typename Ti, typename To, int V, int OP, bool PART, bool NT>
 __global__ __launch_bounds__(kColBlock) void reduce_cols(
     const Ti* __restrict__ x, void* __restrict__ vals, int64_t* __restrict__ idx,
     float* __restrict__ pv, int* __restrict__ pi, int64_t outer, int n, int64_t inner, int cx,
@@ -412,7 +413,7 @@ __global__ __launch_bounds__(kColBlock) void reduce_cols(
   for (; rows - i >= U; i += U, p += U * step) {
     RT v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = load_any<Ti, V>(p + u * step, sx);
+    for (int u = 0; u < U; ++u) v[u] = load_any<Ti, V, NT>(p + u * step, sx);
 #pragma unroll
     for (int u = 0; u < U; ++u) take(v[u], r0 + L.ty + ((i + u) << ty_log2));
   }
@@ -420,7 +421,7 @@ __global__ __launch_bounds__(kColBlock) void reduce_cols(
     RT v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (i + u < rows) v[u] = load_any<Ti, V>(p + u * step, sx);
+      if (i + u < rows) v[u] = load_any<Ti, V, NT>(p + u * step, sx);
 #pragma unroll
     for (int u = 0; u < U; ++u)
       if (i + u < rows) take(v[u], r0 + L.ty + ((i + u) << ty_log2));
@@ -486,6 +487,39 @@ __global__ __launch_bounds__(kColBlock) void reduce_cols(
       write_result<To, 1, OP>(vals, idx, out, r.v, r.i, n, sv, si);
     }
   }
+}
+
+// Short middle axes: one lane per column and no exchange between lanes; bound by
+// latency in the launches that take it (reduce_short_axis in capi.hip has both
+// sides measured).  Consecutive lanes take consecutive columns and a slab's rows
+// lie together, so that the lanes' narrow loads of several rows share lines; they
+// are plain loads, which keep those.  Eight guarded loads in flight per lane were
+// slower (mean bf16 16384 x 2 x 64: 0.77 of the speed, the guards' branches).
+template <typename Ti, typename To, int OP>
+__global__ __launch_bounds__(kColBlock) void reduce_short_cols(const Ti* __restrict__ x,
+                                                               void* __restrict__ vals,
+                                                               int64_t* __restrict__ idx,
+                                                               uint32_t cols, int n,
+                                                               uint32_t inner) {
+  const uint32_t col = blockIdx.x * kColBlock + threadIdx.x;
+  if (col >= cols) return;
+  const uint32_t o = col / inner;
+  const int64_t row = inner;
+  const Ti* xc = x + o * (n * row) + (col - o * inner);
+  const Span sx = VBH_SPAN(x, int64_t(cols) * n);
+  const Span sv = VBH_SPAN(static_cast<To*>(vals), cols), si = VBH_SPAN(idx, cols);
+  auto at = [&](int r) {
+    float f;
+    load_f32<Ti, 1>(xc + r * row, &f, sx);
+    return f;
+  };
+  ValIdx best{OP == 0 ? 0.f : kNegInf, n};
+  for (int r = 0; r < n; ++r) {
+    const float f = at(r);
+    if constexpr (OP == 0) best.v += f;
+    else if (better(f, r, best.v, best.i)) best = ValIdx{f, r};
+  }
+  write_result<To, 1, OP>(vals, idx, col, best.v, best.i, n, sv, si);
 }
 
 // Second stage of a split middle axis: kCombineParts lanes per column, each
@@ -585,13 +619,22 @@ hipError_t launch_reduce_cols(const void* x, void* vals, int64_t* idx, void* par
                       dim3(kColBlock), 0, s, static_cast<const Ti*>(x), vals, idx, pv, pi, outer,
                       n, inner, c.cx, c.ty_log2, static_cast<uint32_t>(c.tiles), c.seg_n);
       };
-      if (c.segs > 1) {
-        launch(reduce_cols<Ti, To, V, OP, true>);
-        launch_kernel((reduce_cols_combine<To, OP>),
-                      dim3(static_cast<uint32_t>((cols + kCombineCols - 1) / kCombineCols)),
-                      dim3(kColBlock), 0, s, pv, pi, vals, idx, cols, n, c.segs);
+      auto tiles = [&](auto nt) {
+        constexpr bool NT = decltype(nt)::value;
+        if (c.segs > 1) launch(reduce_cols<Ti, To, V, OP, true, NT>);
+        else launch(reduce_cols<Ti, To, V, OP, false, NT>);
+      };
+      if (c.short_axis) {
+        launch_kernel((reduce_short_cols<Ti, To, OP>), dim3(static_cast<uint32_t>(c.grid)),
+                      dim3(kColBlock), 0, s, static_cast<const Ti*>(x), vals, idx,
+                      static_cast<uint32_t>(cols), n, static_cast<uint32_t>(inner));
       } else {
-        launch(reduce_cols<Ti, To, V, OP, false>);
+        if (V > 1 && c.nt) tiles(std::bool_constant<(V > 1)>{});
+        else tiles(std::false_type{});
+        if (c.segs > 1)
+          launch_kernel((reduce_cols_combine<To, OP>),
+                        dim3(static_cast<uint32_t>((cols + kCombineCols - 1) / kCombineCols)),
+                        dim3(kColBlock), 0, s, pv, pi, vals, idx, cols, n, c.segs);
       }
       err = hipGetLastError();
     };

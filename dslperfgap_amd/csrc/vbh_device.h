@@ -195,15 +195,17 @@ template <typename T, int V> struct RawAny {
 };
 template <typename T> struct RawAny<T, 1> { typedef T type; };
 
-template <typename T, int V>
+template <typename T, int V, bool NT = true>
 __device__ __forceinline__ typename Raw<T, V>::type load_any(const T* __restrict__ p,
                                                              const Span& s) {
   typedef typename RawAny<T, V>::type A;
   if (!VBH_IN_SPAN(s, p, V * sizeof(T))) return typename Raw<T, V>::type{};
-  return __builtin_nontemporal_load(reinterpret_cast<const A*>(p));
+  const A* q = reinterpret_cast<const A*>(p);
+  if constexpr (NT) return __builtin_nontemporal_load(q);
+  else return *q;
 }
 
-template <typename T, int V>
+template <typename T, int V, bool NT = true>
 __device__ __forceinline__ void store_any(T* __restrict__ p, const float* o, const Span& s) {
   typedef typename RawAny<T, V>::type A;
   if (!VBH_IN_SPAN(s, p, V * sizeof(T))) return;
@@ -214,7 +216,9 @@ __device__ __forceinline__ void store_any(T* __restrict__ p, const float* o, con
 #pragma unroll
     for (int k = 0; k < V; ++k) r[k] = static_cast<T>(o[k]);
   }
-  __builtin_nontemporal_store(r, reinterpret_cast<A*>(p));
+  A* q = reinterpret_cast<A*>(p);
+  if constexpr (NT) __builtin_nontemporal_store(r, q);
+  else *q = r;
 }
 
 // ---------------------------------------------------------------------------

@@ -183,6 +183,8 @@ hipError_t launch_softmax(const void* x, void* y, int64_t rows, int cols, int id
 // `tiles` units per outer slab, `grid` workgroups of `block` lanes.  Reductions:
 // the axis cut into `segs` segments of seg_n rows (the last one shorter).
 // Softmax: `rows` of the axis in registers per lane (0: the streaming kernel).
+// `short_axis`: one lane per column instead (softmax: n <= rows).  `nt`:
+// nontemporal loads (reductions).
 constexpr int kColBlock = 256;
 constexpr int kColMaxSegs = 64;
 struct ColGeometry {
@@ -195,6 +197,8 @@ struct ColGeometry {
   int segs = 1;
   int seg_n = 0;
   int rows = 0;
+  bool short_axis = false;
+  bool nt = true;
 };
 hipError_t launch_softmax_dim(const void* x, void* y, int64_t outer, int n,
                               int64_t inner, int idt, int odt, int log_mode,

@@ -313,6 +313,10 @@ def _special(x):
 
 COL_SHAPES = [(3, n, i) for n in (1, 2, 7, 8, 33) for i in (2, 3, 7, 8, 9, 13, 64, 101)] + [
     (1, 257, 65), (70, 5, 12), (2, 300, 97), (5, 1000, 31), (1, 3000, 2), (600, 40, 68)]
+# one lane per column and, past its limits, tiles: short axes of wide and narrow
+# slabs, large launches
+COL_SHAPES += [(3, n, i) for n in (4, 5, 6, 9, 10, 11, 12, 13, 16, 17) for i in (2, 3, 7, 8, 65)] + [
+    (300, 5, 2000), (70000, 16, 3), (70000, 17, 3), (200000, 6, 2), (90000, 4, 8)]
 # the axis split over workgroups (the last segment shorter in some)
 COL_SPLIT_SHAPES = [(1, 4100, 264), (1, 9001, 33), (2, 20000, 12), (1, 50000, 3)]
 

@@ -258,7 +258,8 @@ def test_split_workspace_sizes():
     assert red(128, 131072, 1, _lib.F32, _lib.REDUCE_MAX) == 128 * 8 * (8 + 4)
     assert red(128, 131072, 1, _lib.F16, _lib.REDUCE_ARGMAX) == 128 * 8 * (8 + 2)
     assert red(300, 131072, 1, _lib.F32, _lib.REDUCE_MEAN) == 0  # long rows: logsumexp only
-    assert red(128, 131072, 4, _lib.F32, _lib.REDUCE_MEAN) == 0  # middle axis: not split
+    assert red(128, 131072, 4, _lib.F32, _lib.REDUCE_MEAN) == 0  # middle axis: enough slabs
+    assert red(1, 4100, 264, _lib.F32, _lib.REDUCE_MEAN) > 0      # one slab of few columns
     sm = h.vbh_softmax_workspace_bytes
     assert sm(128, 131072, _lib.F32) == 128 * 8 * 8       # as logsumexp's few-rows split
     assert sm(8192, 4096, _lib.F32) == 0 and sm(300, 131072, _lib.F32) == 0
