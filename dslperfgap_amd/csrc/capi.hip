@@ -572,8 +572,31 @@ ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int es
 // 16 rows 223).
 constexpr int64_t kSmColUnits = 192;
 
+// Axes of up to 10 (16-bit outputs: 16) run one lane per column
+// (softmax_short_cols) in launches that move up to kSmShortBytes, and beyond that
+// in narrow slabs.  MI355X, log_softmax, device time per call, tiles -> one lane
+// per column: fp16 64 x 2 x 512 4.5 -> 2.6 us, bf16 -> fp32 87381 x 4 x 6
+// 13.1 -> 6.1, fp16 2097152 x 2 x 2 104 -> 12.9, 65536 x 4 x 32 15.8 -> 10.5,
+// 104857 x 10 x 8 24.6 -> 13.2; but fp16 131072 x 4 x 64 31.7 -> 53.3 and fp32
+// 349525 x 8 x 12 49.3 -> 63.5.
+constexpr int64_t kSmShortBytes = int64_t(24) << 20;
+
+bool softmax_short_axis(int64_t outer, int64_t n, int64_t inner, int esize, int osize) {
+  const int size = std::max(esize, osize), vn = 16 / size;
+  if (inner < vn) return n <= (vn == 8 ? 8 : 6);
+  if (n > (vn == 8 ? 16 : 10)) return false;
+  if (mul_sat(mul_sat(outer, inner), n * (esize + osize)) <= kSmShortBytes) return true;
+  return n <= 10 && inner * size <= 96 && n * inner * size <= 256;
+}
+
 ColGeometry softmax_col_geometry(int64_t outer, int64_t n, int64_t inner, int esize, int osize) {
   ColGeometry c;
+  if (softmax_short_axis(outer, n, inner, esize, osize)) {
+    c.short_axis = true;
+    c.rows = n <= 4 ? 4 : n <= 8 ? 8 : 16;
+    c.grid = (mul_sat(outer, inner) + kColBlock - 1) / kColBlock;
+    return c;
+  }
   const int vn = 16 / std::max(esize, osize);
   c.v = inner >= vn ? vn : 1;
   const int64_t cv = (inner + c.v - 1) / c.v;

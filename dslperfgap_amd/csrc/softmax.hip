@@ -7,7 +7,8 @@
 // Streaming path (rows wider than the register budget): one workgroup per row,
 // online (max, rescaled sum) statistics pass, then an output pass.
 // Middle-axis path: contiguous [outer, n, inner] reduced over n, in column
-// tiles: each lane owns the columns of one 16-byte vector and some of the rows.
+// tiles: each lane owns the columns of one 16-byte vector and some of the rows;
+// short axes of small launches or narrow slabs, one lane per column.
 //
 // Semantics: ViperBench/softmax/pytorch_impl.py:4-6 (F.softmax, dim=-1),
 // ViperBench/log_softmax/pytorch_impl.py:4-8 (F.log_softmax(x, dim, dtype)),
@@ -589,11 +590,11 @@ __device__ __forceinline__ void unit_allreduce(float (&v)[V], int cx, int ty_log
 }
 
 // Store V columns at p, less the leading ones the vector before this writes.
-template <typename To, int V>
+template <typename To, int V, bool NT>
 __device__ __forceinline__ void store_cols(To* __restrict__ p, const float (&o)[V], int shared,
                                            const Span& s) {
   if (shared == 0) {
-    store_any<To, V>(p, o, s);
+    store_any<To, V, NT>(p, o, s);
   } else {
 #pragma unroll
     for (int k = 0; k < V; ++k)
@@ -613,6 +614,8 @@ __global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* 
                                                   int64_t outer, int n, int64_t inner, int cx,
                                                   int ty_log2, uint32_t tiles) {
   typedef typename Raw<Ti, V>::type RT;
+  // slabs narrower than a vector: several accesses share each line
+  constexpr bool NT = V > 1;
   __shared__ __align__(16) float lds[2][B / kWave][kColMaxLanes * V];
   const ColLane L = col_lane<V>(outer, inner, cx, ty_log2, tiles);
   const int rows = L.live && L.ty < n ? ((n - L.ty - 1) >> ty_log2) + 1 : 0;  // the lane's
@@ -623,7 +626,7 @@ __global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* 
   const RT fill = RT(static_cast<Ti>(kNegInf));
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    if (i < rows) xr[i] = load_any<Ti, V>(x + at + i * step, sx);
+    if (i < rows) xr[i] = load_any<Ti, V, NT>(x + at + i * step, sx);
     else xr[i] = fill;
   }
   float m[V], s[V];
@@ -654,7 +657,46 @@ __global__ __launch_bounds__(B) void softmax_cols(const Ti* __restrict__ x, To* 
         const float d = raw_at<Ti, V>(xr[i], k) - m[k];
         o[k] = LOG ? d - s[k] : fast_exp(d) * s[k];
       }
-      store_cols<To, V>(y + at + i * step, o, L.shared, sy);
+      store_cols<To, V, NT>(y + at + i * step, o, L.shared, sy);
+    }
+  }
+}
+
+// Short axes (n <= R): one lane per column, its values in registers, no
+// exchange between lanes; plain accesses, since the lanes' narrow loads and
+// stores of several rows share lines.  Bound by latency, or by its narrow accesses
+// (softmax_short_axis in capi.hip has both sides measured).
+template <typename Ti, typename To, int R, bool LOG>
+__global__ __launch_bounds__(kColBlock) void softmax_short_cols(const Ti* __restrict__ x,
+                                                                To* __restrict__ y,
+                                                                uint32_t cols, int n,
+                                                                uint32_t inner) {
+  const uint32_t col = blockIdx.x * kColBlock + threadIdx.x;
+  if (col >= cols) return;
+  const uint32_t o = col / inner;
+  const int64_t row = inner;
+  const int64_t at = o * (n * row) + (col - o * inner);
+  const Span sx = VBH_SPAN(x, int64_t(cols) * n), sy = VBH_SPAN(y, int64_t(cols) * n);
+  float v[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    v[i] = kNegInf;
+    if (i < n) load_f32<Ti, 1>(x + at + i * row, &v[i], sx);
+  }
+  float m = v[0];
+#pragma unroll
+  for (int i = 1; i < R; ++i) m = max_nan(m, v[i]);
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+    if (i < n) s += fast_exp(v[i] - m);
+  s = LOG ? fast_log(s) : 1.0f / s;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i < n) {
+      const float d = v[i] - m;
+      const float out = LOG ? d - s : fast_exp(d) * s;
+      store_from_f32<To, 1>(y + at + i * row, &out, sy);
     }
   }
 }
@@ -730,7 +772,7 @@ __global__ __launch_bounds__(B) void softmax_cols_stream(const Ti* __restrict__ 
           const float d = raw_at<Ti, V>(v[u], k) - gm[k];
           o[k] = LOG ? d - s[k] : fast_exp(d) * s[k];
         }
-        store_cols<To, V>(y + at + (i + u) * step, o, L.shared, sy);
+        store_cols<To, V, true>(y + at + (i + u) * step, o, L.shared, sy);
       }
     }
   }
@@ -916,7 +958,16 @@ hipError_t launch_softmax_dim(const void* x, void* y, int64_t outer, int n, int6
     auto go = [&](auto vc, auto lc) {
       constexpr int V = decltype(vc)::value;
       constexpr bool LOG = decltype(lc)::value;
-      if (c.rows == 0) launch(softmax_cols_stream<Ti, To, V, LOG, kMaxBlock>);
+      auto short_axis = [&](auto kern) {
+        launch_kernel(kern, dim3(static_cast<uint32_t>(c.grid)), dim3(kColBlock), 0, s,
+                      static_cast<const Ti*>(x), static_cast<To*>(y),
+                      static_cast<uint32_t>(outer * inner), n, static_cast<uint32_t>(inner));
+        err = hipGetLastError();
+      };
+      if (c.short_axis && c.rows == 4) short_axis(softmax_short_cols<Ti, To, 4, LOG>);
+      else if (c.short_axis && c.rows == 8) short_axis(softmax_short_cols<Ti, To, 8, LOG>);
+      else if (c.short_axis) short_axis(softmax_short_cols<Ti, To, 16, LOG>);
+      else if (c.rows == 0) launch(softmax_cols_stream<Ti, To, V, LOG, kMaxBlock>);
       else if (c.rows == 4) launch(softmax_cols<Ti, To, V, 4, LOG, kColBlock>);
       else if (c.rows == 8 && c.block == kColBlock) launch(softmax_cols<Ti, To, V, 8, LOG, kColBlock>);
       else if (c.rows == 8) launch(softmax_cols<Ti, To, V, 8, LOG, kMaxBlock>);

@@ -1,7 +1,8 @@
 """GPU parity of softmax / log_softmax over a middle axis (column tiles): every
 launch shape of the kernel -- 4, 8 and 16 rows per lane in 256 lanes, 8 and 16
-in 1024, the streaming one; 16, 8, 4, 2 and 1 lanes per line; vectors moved back
-at a slab's edge -- against the oracle.
+in 1024, the streaming one, each at 8 lanes per line; 16, 4, 2 and 1 lanes per
+line as well; vectors moved back at a slab's edge -- and short axes with one lane
+per column (4, 8 and 16 values per lane), against the oracle.
 """
 import pytest
 import torch
@@ -20,7 +21,15 @@ TOL = {torch.float32: 1e-5, torch.float16: 2e-3, torch.bfloat16: 1.6e-2}
 
 SHAPES = [(3, n, i) for n in (1, 2, 4, 5, 33, 64, 65) for i in (2, 5, 8, 13, 64, 130)] + [
     (200, 3, 136), (200, 40, 136), (2, 513, 33), (30, 500, 64), (1, 1025, 40), (100, 1024, 16),
-    (3, 2049, 9), (200, 2048, 8), (1, 9000, 20), (200, 2300, 9)]
+    (3, 2049, 9), (200, 2048, 8), (1, 9000, 20), (200, 2300, 9),
+    # 8 and 16 lanes per line: 8 and 16 rows per lane in 256 lanes, then 8 and 16
+    # rows in 1024, streaming; the smallest that the rule sends to each
+    (260, 33, 257), (260, 33, 520), (260, 17, 520), (200, 129, 17), (100, 65, 65),
+    (200, 513, 17), (200, 1025, 17), (200, 2049, 17), (200, 9000, 3), (1, 2049, 2), (1, 2049, 3)]
+# one lane per column at every count of values per lane, and beyond it (narrow slabs
+# of more than 6 or 8, the others of more than 10 or 16); a large launch in tiles
+SHAPES += [(3, n, i) for n in (3, 6, 7, 8, 9, 10, 11, 16, 17) for i in (2, 3, 7, 13, 65)] + [
+    (400, 8, 1024), (70000, 10, 12)]
 
 
 def _input(shape, dtype):
@@ -45,6 +54,11 @@ def test_middle_axis_softmax(shape, dtype, out):
     xd = x.to(DEV)
     tol = TOL[out or dtype]
     got, want = log_softmax(xd, 1, out).cpu(), ref.log_softmax(x, 1, out)
+    if shape[1] > 4096 and want.dtype == torch.float32:
+        # the oracle adds up a column's exps one after the other in 32 bits: over
+        # 9000 of them it is up to 1.39 of this tolerance off the result in 64 bits
+        # (200 x 9000 x 3, these inputs)
+        want = torch.log_softmax(x.double(), 1).float()
     assert got.dtype == want.dtype and got.shape == want.shape
     assert torch.allclose(got.float(), want.float(), atol=tol, rtol=tol, equal_nan=True)
     # softmax over a middle axis is reached through the C ABI only
