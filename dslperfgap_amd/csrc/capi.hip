@@ -59,6 +59,13 @@ std::atomic<int> g_tpr[kNumOps];
 std::atomic<int> g_block[kNumOps];
 std::atomic<int> g_flags[kNumOps];
 
+// a * b for sizes (a, b >= 0), saturated at INT64_MAX: products of caller
+// sizes are formed before the range checks that reject them.
+int64_t mul_sat(int64_t a, int64_t b) {
+  int64_t r;
+  return __builtin_mul_overflow(a, b, &r) ? INT64_MAX : r;
+}
+
 // Built-in choices per op, from launch-shape sweeps on MI355X:
 //   vectors per lane before more lanes are added (pick_geometry): 2 for RMSNorm
 //   and fp32 softmax, 4 for 16-bit softmax (bf16 8192 columns: +8% over 2),
@@ -99,7 +106,18 @@ constexpr int64_t kShortRowVecs = 32;
 constexpr int kItShort[kNumOps] = {2, 2, 2, 2, 4, 4};
 constexpr int kMinLanesShort[kNumOps] = {4, 8, 8, 8, 2, 4};
 
-int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in) {
+// 16-bit softmax rows written as fp32 (8-byte vectors): launches of this many
+// elements or more choose by row width more finely (it_target, mixed_eight)
+constexpr int64_t kMixedManyElems = int64_t(1) << 21;
+
+int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in, int64_t units) {
+  // 16-bit softmax rows written as fp32, 9-12 vectors: 8 lanes of 2, and 16 lanes
+  // of 1 only in small launches.  MI355X, 16 -> 8 lanes, fp16 / bf16 at 2^25
+  // elements: 36 columns 59.0 -> 42.3 / 61.4 -> 42.3 us, 44 columns 52.2 -> 44.4 /
+  // 52.9 -> 45.3; at 2^20 3.68 -> 3.87 / 3.79 -> 3.98.
+  if (op == VBH_OP_SOFTMAX && half_in && vec == 4 && nvec > 8 && nvec <= 12 &&
+      mul_sat(units, nvec * vec) >= kMixedManyElems)
+    return 2;
   if (vec > 1 && nvec <= kShortRowVecs) {
     int it = kItShort[op];
     while (it > 1 && nvec / it < kMinLanesShort[op]) it /= 2;
@@ -111,6 +129,14 @@ int it_target(int op, int64_t nvec, int vec, bool column_blocks, bool half_in) {
   // the 8-byte vectors of 16-bit rows written as fp32 (bf16 20000 x 255 at 1 / 2
   // / 4 vectors 9.6 / 9.0 / 7.3 us, fp16 50000 x 135 17.2 / 12.8 / 12.7)
   if (op == VBH_OP_SOFTMAX && vec == 4 && nvec <= kWave) return half_in ? 4 : 1;
+  // and 4 of them from 129 vectors up, but 2 in rows of up to 512 that fill every
+  // wave at 2 (fp16 2^23 / 2^25 elements, us at 2 -> 4 per lane: 569 columns
+  // 15.4 -> 11.4 / 53.9 -> 36.8, 2560 11.1 -> 10.6 / 37.7 -> 33.8, 4096
+  // 10.4 -> 8.5 / 34.6 -> 34.4, 8192 11.0 -> 8.3 / 40.4 -> 34.6; but 448 columns
+  // 10.2 -> 10.8 / 32.3 -> 34.1 and 1024 9.9 -> 8.5 / 32.8 -> 34.6)
+  if (op == VBH_OP_SOFTMAX && vec == 4 && half_in && nvec > 2 * kWave &&
+      !(nvec <= 8 * kWave && nvec % (2 * kWave) == 0))
+    return 4;
   // 16-bit LayerNorm rows of 1025-1536 vectors: 2 vectors per lane, 9-12 waves
   // per row (bf16 at 64 MB per call, 4 -> 2: 9216 columns 4298 -> 5247 GB/s,
   // 10240 4501 -> 5194, 11264 4855 -> 5199, 12288 5126 -> 5290; at 768 and
@@ -165,13 +191,6 @@ int pow2ceil(int64_t n) {
   int p = 1;
   while (p < n) p <<= 1;
   return p;
-}
-
-// a * b for sizes (a, b >= 0), saturated at INT64_MAX: products of caller
-// sizes are formed before the range checks that reject them.
-int64_t mul_sat(int64_t a, int64_t b) {
-  int64_t r;
-  return __builtin_mul_overflow(a, b, &r) ? INT64_MAX : r;
 }
 
 int row_group_lanes(int64_t nvec, int it) {
@@ -331,7 +350,8 @@ Geometry geometry_for(int op, int64_t cols, int vec, int64_t units, int64_t out_
   const int64_t nvec = cols / vec;
   const bool half_in = dtype == kF16 || dtype == kBF16;
   Geometry g =
-      pick_geometry(cols, vec, fill_it(it_target(op, nvec, vec, column_blocks, half_in), nvec, units),
+      pick_geometry(cols, vec,
+                    fill_it(it_target(op, nvec, vec, column_blocks, half_in, units), nvec, units),
                     g_tpr[op].load(), g_block[op].load(), flags);
   if (g.persist && !(over & kFlagPersist) && g.tpr < kPersistMinTpr[op]) g.persist = false;
   // LayerNorm row groups of exactly 2 waves run 4 to a 512-lane workgroup
@@ -421,7 +441,8 @@ Geometry reduce_geometry(int64_t n, int vec, int64_t units) {
   const int64_t nvec = n / vec;
   int tpr = g_tpr[VBH_OP_REDUCE].load();
   if (tpr <= 0) {
-    const int per_lane = fill_it(it_target(VBH_OP_REDUCE, nvec, vec, false, false), nvec, units);
+    const int per_lane =
+        fill_it(it_target(VBH_OP_REDUCE, nvec, vec, false, false, units), nvec, units);
     const int64_t lanes = (nvec + per_lane - 1) / per_lane;
     if (lanes <= kWave) {
       tpr = pow2ceil(lanes < 1 ? 1 : lanes);
@@ -971,6 +992,26 @@ RowSplit softmax_split(int64_t rows, int64_t cols, int vn) {
   return RowSplit{static_cast<int>((cols + seg_cols - 1) / seg_cols), seg_cols};
 }
 
+namespace {
+
+// Whether 16-bit rows written as fp32 take 8 elements per lane access after all:
+// short rows that then have one access per lane and half the lanes, in launches
+// of kMixedManyElems or more.  MI355X, 4 -> 8 elements, fp16 / bf16 at 2^25
+// elements: 24 columns 48.3 -> 38.4 / 50.6 -> 39.1 us, 40 54.3 -> 38.8 /
+// 57.3 -> 39.7, 56 43.6 -> 37.7 / 45.1 -> 38.8, 41 69.0 -> 54.6 / 74.1 -> 58.0,
+// 65 60.8 -> 51.9 / 58.6 -> 52.0 (at 2^23 14.4 -> 15.7), at 2^22 40 9.0 -> 7.6 /
+// 9.0 -> 7.5; but 64 34.5 -> 38.5 / 34.0 -> 38.9, 35 50.1 -> 56.7 /
+// 52.5 -> 61.3, 52 45.5 -> 48.2 / 47.3 -> 48.5 and, at 2^20, 24 columns 3.53 -> 3.77.
+bool mixed_eight(int64_t rows, int64_t cols) {
+  const int64_t elems = mul_sat(rows, cols);
+  if (g_tpr[VBH_OP_SOFTMAX].load() || g_block[VBH_OP_SOFTMAX].load() || elems < kMixedManyElems)
+    return false;
+  if (cols % 8 == 0) return cols >= 24 && cols < 64;
+  return cols % 4 != 0 && cols > 36 && cols < (elems < 8 * kMixedManyElems ? 64 : 68);
+}
+
+}  // namespace
+
 int64_t vbh_softmax_workspace_bytes(int64_t rows, int64_t cols, int in_dtype) {
   if (!is_float(in_dtype) || rows <= 0 || cols <= 0 || cols > kMaxCols) return 0;
   const int vn = 16 / elt_size(in_dtype);
@@ -995,7 +1036,8 @@ int vbh_softmax_fwd_ws(const void* x, void* y, int64_t rows, int64_t cols, int i
   if (rows == 0 || cols == 0) return 0;
   if (!x || !y) return fail(VBH_E_INVALID, "softmax: null pointer");
   const int vn = 16 / elt_size(in_dtype);
-  const int vo = std::min(vn, 16 / elt_size(out_dtype));  // of the kernels that write y
+  // elements per lane access of the kernels that write y
+  const int vo = mixed_eight(rows, cols) ? vn : std::min(vn, 16 / elt_size(out_dtype));
   const bool aligned = aligned16(x) && aligned16(y);
   const bool vec_ok = cols % vo == 0 && aligned;
   const bool mis_ok = !vec_ok && aligned && cols >= kMisMinVecs * vo;

@@ -117,7 +117,8 @@ __device__ __forceinline__ MisRow mis_row(int64_t start, int cols) {
 // lie side by side; with 8 elements per lane every store left 16-byte gaps for
 // the next one (MI355X, bf16 -> fp32
 // log_softmax, 8 -> 4 elements: 1024 x 50257 91 -> 71 us, 8192 x 4096 52.6 -> 33.5,
-// 512 x 65536 68 -> 40).
+// 512 x 65536 68 -> 40).  Some short rows keep 8, one access per lane (mixed_eight
+// in capi.hip).
 template <typename Ti, typename To>
 constexpr int softmax_vec = Vec<To>::n < Vec<Ti>::n ? Vec<To>::n : Vec<Ti>::n;
 
@@ -799,18 +800,22 @@ hipError_t launch_softmax(const void* x, void* y, int64_t rows, int cols, int id
     using Ti = typename decltype(ti)::type;
     using To = typename decltype(to)::type;
     constexpr int VN = softmax_vec<Ti, To>;
+    // 16-bit rows written as fp32 with 8 elements per lane access: one access per lane
+    constexpr int kWide = Vec<Ti>::n;
     auto go = [&](auto vc, auto lc) {
       constexpr int V = decltype(vc)::value;
       constexpr bool LOG = decltype(lc)::value;
-      if (g.stream) {
-        launch_kernel((softmax_stream<Ti, To, V, LOG>), dim3(rows), dim3(g.block), 0, s,
-                           static_cast<const Ti*>(x), static_cast<To*>(y), cols);
-        err = hipGetLastError();
-        return;
+      if constexpr (V <= VN) {
+        if (g.stream) {
+          launch_kernel((softmax_stream<Ti, To, V, LOG>), dim3(rows), dim3(g.block), 0, s,
+                             static_cast<const Ti*>(x), static_cast<To*>(y), cols);
+          err = hipGetLastError();
+          return;
+        }
       }
       dispatch_maxit(g.maxit, [&](auto mc) {
         constexpr int M = decltype(mc)::value;
-        if constexpr (M <= lane_cap(V)) {
+        if constexpr (M <= lane_cap(V) && (V <= VN || M == 1)) {
           dispatch_store_policy<V>(g, [&](auto sp) {
             constexpr int SP = decltype(sp)::value;
             if (V > 1 && g.mis)
@@ -833,6 +838,7 @@ hipError_t launch_softmax(const void* x, void* y, int64_t rows, int cols, int id
       else go(vc, std::false_type{});
     };
     if (g.v == 1) with_log(std::integral_constant<int, 1>{});
+    else if (g.v == kWide) with_log(std::integral_constant<int, kWide>{});
     else with_log(std::integral_constant<int, VN>{});
   });
   return err;

@@ -1,6 +1,7 @@
 """GPU parity of the softmax row kernels' vector shapes: 16-bit rows written as
 fp32 (4 elements per lane access: row widths around multiples of 4 and 8, one
-vector, one wave, several waves, the streaming kernel, split rows), fp32 softmax
+vector, one wave, several waves, the streaming kernel, split rows; 8 elements in
+large launches of short rows), fp32 softmax
 rows of 64 values per lane (near and far from 0), and streaming rows of every
 type with special values, against torch in 64 bits: over rows this long the
 oracle's own 32-bit sums are up to 1.7e-5 off (an output of -0.5582618 in 64 bits
@@ -46,7 +47,13 @@ def _close(got, want, dtype, what):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,cols", [(33, c) for c in (1, 7, 16, 17, 20, 132, 255, 256, 260, 1001,
                                                          4096, 4098, 16389, 50257)]
-                         + [(200, 65540), (140, 131072), (4, 50257), (3, 131075)])
+                         + [(200, 65540), (140, 131072), (4, 50257), (3, 131075)]
+                         # 2, 4 vectors per lane
+                         + [(33, c) for c in (516, 569, 1024, 1028, 2560, 5824)]
+                         # large launches of short rows: 8 elements per access at
+                         # 24 to 56 and 37 to 67 columns, 4 beside them
+                         + [(2**22 // c + 1, c) for c in (23, 24, 32, 36, 37, 40, 41, 44, 47, 48,
+                                                          52, 55, 56, 63, 64, 65, 67, 69)])
 def test_16_bit_rows_to_fp32(rows, cols, dtype):
     x = _rows(rows, cols, dtype)
     _close(log_softmax(x.to(DEV), -1, torch.float32), torch.log_softmax(x.double(), -1),
