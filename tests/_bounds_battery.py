@@ -1,8 +1,9 @@
 """A battery of calls that reaches every kernel of libvbhip at least once:
 each row kernel (register-resident, persistent guarded and unguarded,
-streaming, rows that are not whole vectors), the split first and second
-stages, the middle-axis kernels, the cross-entropy forward / combine /
-backward, the no-allocation entry point and the copy / read yardsticks.
+streaming, rows that are not whole vectors, 16-bit rows written as fp32), the
+split first and second stages, the middle-axis kernels (one lane per column,
+tiles, split, streaming), the cross-entropy forward (rows, streaming, persistent,
+any-row) / combine / backward, the no-allocation entry point and the copy / read yardsticks.
 
 ``run()`` returns {case name: output tensor on the CPU}.  The debug-bounds
 test runs it once under the release library (in the pytest process) and once
@@ -83,12 +84,27 @@ def run() -> dict:
         out[f"softmax {key}"] = softmax(x)
         out[f"log_softmax {key}"] = log_softmax(x)
         out[f"logsumexp {key}"] = logsumexp(x)
+    # 16-bit rows written as fp32: rows (whole vectors and not, 8 elements per
+    # access), split, streaming
+    for rows, cols in ((33, 256), (33, 1001), (110000, 40), (110000, 41), (4, 50257), (200, 65540),
+                       (200, 65541)):
+        x = _x(rows, cols, 7, torch.bfloat16, 3.0)
+        out[f"log_softmax {rows}x{cols} bf16 to fp32"] = log_softmax(x, 1, torch.float32)
+    # middle axes: one lane per column (narrow and wide slabs), tiles whose last
+    # vector is moved back, tiles of several waves, streaming; plain and
+    # nontemporal accesses
+    for shape in ((6, 40, 24), (3, 5, 7), (5, 9, 200), (3, 33, 2), (3, 33, 13), (260, 33, 257),
+                  (2, 600, 130), (2, 2049, 9), (2, 9000, 9)):
+        x3 = (3 * torch.randn(shape, generator=_g(8))).to(DEV)
+        key = "x".join(map(str, shape))
+        out[f"log_softmax {key} dim 1"] = log_softmax(x3, 1)
+        out[f"log_softmax {key} dim 1 fp16"] = log_softmax(x3.half(), 1)
+        out[f"log_softmax {key} dim 1 fp16 to fp32"] = log_softmax(x3.half(), 1, torch.float32)
     x3 = (3 * torch.randn(6, 40, 24, generator=_g(8))).to(DEV)
-    out["log_softmax dim 1"] = log_softmax(x3, 1)
     out["log_softmax dim 0 fp32 out"] = log_softmax(x3.half(), 0, torch.float32)
     out["logsumexp 600x70000"] = logsumexp(_x(600, 70000, 9, scale=2.0))
     # cross entropy forward: column blocks, labels int32 / int64, rows not whole
-    # vectors, split rows (segments + combine), streaming segments; backward tiles
+    # vectors, split rows (segments + combine), long rows (any-row); backward tiles
     for rows, cols, bs, ldt in ((64, 1000, 256, torch.int64), (33, 1001, 1024, torch.int32),
                                 (7, 131072, 131072, torch.int64),
                                 (5, 131075, 131075, torch.int32),
@@ -105,6 +121,26 @@ def run() -> dict:
             n = rows * -(-cols // bs)
             for i, t in enumerate(res):
                 out[f"ce {rows}x{cols} bs{bs} sm{sm} out{i}"] = t.reshape(-1)[:n].clone()
+    # rows beyond the registers that are neither split nor the any-row kernel's
+    logits = _x(256, 70000, 10, torch.bfloat16, 2.0)
+    labels = torch.randint(0, 70000, (256,), generator=_g(11)).to(DEV)
+    res = cross_entropy_fwd(logits, labels, 0.1, 0.9, 0.01, -100, 70000, 0, 70000, True, False)
+    for i, t in enumerate(res):
+        out[f"ce 256x70000 bf16 out{i}"] = t.reshape(-1)[:256].clone()
+    # the any-row forward: rows off the vector boundary in a buffer that is off
+    # it too, with and without gaps between them
+    for rows, cols, dt, pad, offset in ((520, 36864, torch.bfloat16, 3, 5),
+                                        (513, 32776, torch.float16, 0, 1),
+                                        (1100, 32771, torch.float32, 0, 3)):
+        store = torch.zeros(offset + rows * (cols + pad) - pad, dtype=dt, device=DEV)
+        logits = store[offset:].as_strided((rows, cols), (cols + pad, 1))
+        logits.copy_(_x(rows, cols, 10, dt, 2.0))
+        labels = torch.randint(0, cols, (rows,), generator=_g(11)).to(DEV)
+        for sm in (0.0, 0.1):
+            res = cross_entropy_fwd(logits, labels, sm, 1.0, 0.01, -100, cols, 0, cols, sm > 0,
+                                    False)
+            for i, t in enumerate(res):
+                out[f"ce any {rows}x{cols} {dt} sm{sm} out{i}"] = t.reshape(-1)[:rows].clone()
     # the persistent forward (forced: a few rows, the last chunk of a row partly
     # past its end, int32 labels, smoothing; workgroups of 256 and 512 lanes)
     rows, cols = 40, 20000
@@ -147,6 +183,17 @@ def run() -> dict:
         out[f"argmax {key}"] = argmax(x, 1)
         out[f"mean dim0 {key}"] = mean_reduction(x, 0)
         out[f"argmax dim0 {key}"] = argmax(x, 0)
+    # middle axes: one lane per column, tiles whose last vector is moved back,
+    # whole memory lines, the axis split over workgroups
+    for shape in ((3, 5, 7), (5, 9, 200), (3, 33, 3), (3, 33, 13), (30, 40, 256), (1, 9001, 33),
+                  (1, 4100, 264)):
+        x3 = (3 * torch.randn(shape, generator=_g(20))).to(DEV)
+        for dt in (torch.float32, torch.bfloat16):
+            key = "x".join(map(str, shape)) + f" {dt}"
+            out[f"mean {key}"] = mean_reduction(x3.to(dt), 1)
+            out[f"max {key}"], out[f"max idx {key}"] = max_reduction(x3.to(dt), 1)
+            out[f"argmax {key}"] = argmax(x3.to(dt), 1)
+        out[f"mean {key} to fp32"] = mean_reduction(x3.to(dt), 1, False, torch.float32)
     # the yardsticks
     nbytes = 1 << 20
     src = torch.randint(0, 1 << 30, (nbytes // 4,), generator=_g(18), dtype=torch.int32).to(DEV)

@@ -243,6 +243,27 @@ def test_any_row_cross_entropy_matches_oracle(dtype, rows, cols, pad, offset, pi
     _check(got, ref.cross_entropy_fwd(logits, labels, **args), rows, f"any {rows}x{cols} {dtype}")
 
 
+@pytest.mark.parametrize("cols,pi", [(32773, 1), (36864, 0)])
+def test_any_row_cross_entropy_workgroups_walk_rows(cols, pi):
+    """fp32 launches give each of the resident workgroups (two per CU) equal
+    shares: 1400 rows on 512 workgroups three rows each, the last round partly
+    filled.  A row's maximum differs from its neighbours', and the rows with
+    special values come last."""
+    rows = 1400
+    logits, labels = _inputs(rows, cols, torch.float32, 980 + pi, 0)
+    r = torch.arange(12, rows)
+    logits[r, (r * 97) % cols] += 10.0 + (r % 13).float()
+    logits, labels = logits.flip(0), labels.flip(0)
+    args = dict(ignored_index=-100, total_classes=cols, class_start_idx=0, BLOCK_SIZE=cols,
+                **PARAMS[pi])
+    print(f"[ce persist] walk {rows}x{cols} params {pi}", flush=True)
+    store = torch.empty(rows * (cols + 1), device=DEV)
+    xd = store.view(rows, cols + 1)[:, :cols]  # rows off the 16-byte boundary
+    xd.copy_(logits)
+    got = cross_entropy_fwd(xd, labels.to(DEV), **args)
+    _check(got, ref.cross_entropy_fwd(logits, labels, **args), rows, f"walk {rows}x{cols}")
+
+
 # which kernel takes aligned 16-bit rows without smoothing of 12 or 16 of
 # ce_fwd_rows' waves (4096 columns each): True where that kernel keeps them
 KEPT = [(torch.bfloat16, 2048, 65536, True), (torch.bfloat16, 2047, 65536, False),
