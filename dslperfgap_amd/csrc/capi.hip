@@ -578,13 +578,17 @@ ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int es
 
 // Launch shape of a middle-axis softmax over [outer, n, inner] (esize / osize
 // bytes per element of input and output).  8 lanes per line (a 128-byte line of
-// memory), 16 where a vector is 8 bytes of input or a lane holds the whole axis;
-// 4, or 2, where that leaves
-// fewer than kSmColUnits units, though two units then fetch each line.  MI355X,
-// log_softmax over the middle axis, us: bf16 -> fp32 16 x 64 x 16384 at 8 / 16
-// lanes 22.8 / 18.9; bf16 8 x 1000 x 1024 (128 units) at 8 / 4 19.4 / 15.5,
-// bf16 4 x 4096 x 1024 60 / 33.5, but fp32 8 x 2000 x 1024 (256 units)
-// 27.7 / 42.
+// memory), 16 where a vector is 8 bytes of input or a lane holds the whole axis,
+// unless that leaves fewer than kSmColUnits units; 4 below kSmColUnits4 units (and
+// then 2 of an axis that would stream), though two units then fetch each line.
+// MI355X, log_softmax over the middle axis, us: bf16 -> fp32 16 x 64 x 16384 at 8 / 16
+// lanes 22.8 / 18.9; at 8 / 4 lanes, by units of 8 lanes (8 slabs):
+//   units             128           160           192           256
+//   bf16 n = 300    9.1 / 9.7     9.3 / 9.5     9.3 / 9.4     9.4 / 9.7
+//   bf16 1000      18.0 / 14.5   18.6 / 18.9   19.2 / 21.6   20.6 / 23.8
+//   bf16 4000      67.3 / 45.3   66.7 / 73.3   78.0 / 78.5   92.3 / 88.9
+//   fp32 1000      11.2 / 10.9   12.0 / 17.8   13.2 / 22.4   15.0 / 25.4
+//   fp32 4000      59.5 / 48.5   58.8 / 61.3   70.7 / 79.2   87.4 / 96.2
 // Rows per lane: up to a wave per unit 4 or 8, then 16 in 256-lane workgroups
 // (fp16 64 x 512 x 768: 19.1, 8 rows in 1024 lanes 32.4; fp32 64 x 150 x 2048
 // 30.9 against 32.9), 4 while the launch has fewer than 512 workgroups, 8 and
@@ -592,6 +596,7 @@ ColGeometry col_geometry(int64_t outer, int64_t n, int64_t inner, int vn, int es
 // Axes that do not fit at 8 lanes stream (fp32 2 x 4096 x 8192: 170, 4 lanes of
 // 16 rows 223).
 constexpr int64_t kSmColUnits = 192;
+constexpr int64_t kSmColUnits4 = 144;
 
 // Axes of up to 10 (16-bit outputs: 16) run one lane per column
 // (softmax_short_cols) in launches that move up to kSmShortBytes, and beyond that
@@ -629,7 +634,7 @@ ColGeometry softmax_col_geometry(int64_t outer, int64_t n, int64_t inner, int es
   c.cx = 16;
   if (n > 4 && (c.v * esize == 16 || !fits(16, kColBlock) || units() < kSmColUnits))
     c.cx = 8;
-  if (n > kWave && units() < kSmColUnits) c.cx = 4;
+  if (n > kWave && units() < kSmColUnits4) c.cx = 4;
   if (c.cx == 4 && !fits(16, kMaxBlock) && units() < kSmColUnits) c.cx = 2;
   c.cx = static_cast<int>(std::min<int64_t>(pow2ceil(cv), c.cx));
   c.tiles = (cv + c.cx - 1) / c.cx;

@@ -125,7 +125,7 @@ constexpr int softmax_vec = Vec<To>::n < Vec<Ti>::n ? Vec<To>::n : Vec<Ti>::n;
 // The row's exp form for softmax of fp32 rows of 64 values per lane: both forms
 // of ExpFma and ExpSub in one, 2^((x - m1) * log2 e - mb) with m1 = 0 or mb = 0,
 // for a subtract per element.  With the two forms beside each other the
-// kernel's 128 VGPRs did not hold the row (42-59 of them spilled).  MI355X,
+// kernel's 128 VGPRs did not hold the row (42-61 of them spilled).  MI355X,
 // softmax fp32 1000 x 65536 130 -> 104 us, 2048 x 50257 191 -> 167.
 struct ExpEither {
   float m1, mb;
