@@ -1015,6 +1015,15 @@ bool mixed_eight(int64_t rows, int64_t cols) {
   return cols % 4 != 0 && cols > 36 && cols < (elems < 8 * kMixedManyElems ? 64 : 68);
 }
 
+// Split 16-bit rows written as fp32: the second stage takes 8 elements per lane
+// access in launches between these, where half the workgroups weigh more than the
+// gaps between the stores.  MI355X, 4 -> 8 elements, both stages, us: fp16
+// 16 x 120987 8.2 -> 8.0, 32 x 120987 11.5 -> 10.7, 64 x 50257 10.3 -> 9.6,
+// 64 x 100000 15.1 -> 14.5, 64 x 131072 17.8 -> 17.7; but 16 x 65536 5.9 -> 6.3,
+// 4 x 131072 6.0 -> 6.2 and 128 x 100000 22.7 -> 26.3.
+constexpr int64_t kMixedApplyMinElems = int64_t(7) << 18;
+constexpr int64_t kMixedApplyMaxElems = int64_t(1) << 23;
+
 }  // namespace
 
 int64_t vbh_softmax_workspace_bytes(int64_t rows, int64_t cols, int in_dtype) {
@@ -1059,8 +1068,10 @@ int vbh_softmax_fwd_ws(const void* x, void* y, int64_t rows, int64_t cols, int i
     const int64_t units = rows * segs;
     const int seg_cols = static_cast<int>(sp.seg_cols);
     Geometry g1 = geometry_for(VBH_OP_LOGSUMEXP, seg_cols, vn, units);
-    Geometry g2 = geometry_for(VBH_OP_SOFTMAX, cols, vo, rows, out_bytes);  // nt / wt
-    g2.mis = !vec_ok;
+    const int64_t elems = mul_sat(rows, cols);
+    const int va = elems >= kMixedApplyMinElems && elems <= kMixedApplyMaxElems ? vn : vo;
+    Geometry g2 = geometry_for(VBH_OP_SOFTMAX, cols, va, rows, out_bytes);  // nt / wt
+    g2.mis = cols % va != 0;
     const bool even = cols % vn == 0;
     if (even || use_mis(g1, vn)) {
       if (int rc = check_grid(units, g1)) return rc;

@@ -926,23 +926,27 @@ hipError_t launch_softmax_apply(const void* x, void* y, const float* seg_pairs, 
   dispatch_in_out(idt, odt, [&](auto ti, auto to) {
     using Ti = typename decltype(ti)::type;
     using To = typename decltype(to)::type;
-    constexpr int V = softmax_vec<Ti, To>;
-    const int64_t tiles = (cols / V + kApplyLanes - 1) / kApplyLanes;
-    dispatch_store_policy<V>(g, [&](auto sp) {
-      constexpr int SP = decltype(sp)::value;
-      auto launch = [&](auto kern) {
-        launch_kernel(kern, dim3(rows * tiles), dim3(kApplyLanes), 0, s,
-                           static_cast<const Ti*>(x), static_cast<To*>(y), seg_pairs, cols, segs,
-                           static_cast<uint32_t>(tiles));
-      };
-      if (g.mis) {
-        if (log_mode) launch(softmax_apply_tiles<Ti, To, V, true, SP, true>);
-        else launch(softmax_apply_tiles<Ti, To, V, false, SP, true>);
-      } else {
-        if (log_mode) launch(softmax_apply_tiles<Ti, To, V, true, SP, false>);
-        else launch(softmax_apply_tiles<Ti, To, V, false, SP, false>);
-      }
-    });
+    auto go = [&](auto vc) {
+      constexpr int V = decltype(vc)::value;
+      const int64_t tiles = (cols / V + kApplyLanes - 1) / kApplyLanes;
+      dispatch_store_policy<V>(g, [&](auto sp) {
+        constexpr int SP = decltype(sp)::value;
+        auto launch = [&](auto kern) {
+          launch_kernel(kern, dim3(rows * tiles), dim3(kApplyLanes), 0, s,
+                             static_cast<const Ti*>(x), static_cast<To*>(y), seg_pairs, cols, segs,
+                             static_cast<uint32_t>(tiles));
+        };
+        if (g.mis) {
+          if (log_mode) launch(softmax_apply_tiles<Ti, To, V, true, SP, true>);
+          else launch(softmax_apply_tiles<Ti, To, V, false, SP, true>);
+        } else {
+          if (log_mode) launch(softmax_apply_tiles<Ti, To, V, true, SP, false>);
+          else launch(softmax_apply_tiles<Ti, To, V, false, SP, false>);
+        }
+      });
+    };
+    if (g.v == Vec<Ti>::n) go(std::integral_constant<int, Vec<Ti>::n>{});
+    else go(std::integral_constant<int, softmax_vec<Ti, To>>{});
     err = hipGetLastError();
   });
   return err;

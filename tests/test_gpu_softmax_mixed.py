@@ -48,6 +48,8 @@ def _close(got, want, dtype, what):
 @pytest.mark.parametrize("rows,cols", [(33, c) for c in (1, 7, 16, 17, 20, 132, 255, 256, 260, 1001,
                                                          4096, 4098, 16389, 50257)]
                          + [(200, 65540), (140, 131072), (4, 50257), (3, 131075)]
+                         # split, on both sides of 7 * 2^18 and 2^23 elements
+                         + [(14, 131072), (13, 131072), (64, 131072), (65, 131072), (40, 120987)]
                          # 2, 4 vectors per lane
                          + [(33, c) for c in (516, 569, 1024, 1028, 2560, 5824)]
                          # large launches of short rows: 8 elements per access at
